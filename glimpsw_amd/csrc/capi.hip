@@ -99,6 +99,10 @@ struct Scratch {
     uint32_t* bin_order = nullptr;
     size_t bin_order_cap = 0;
     size_t bin_lists_cap = 0;
+    uint32_t* coarse_counts = nullptr; // cleared by each launch's cull
+    size_t coarse_counts_cap = 0;
+    uint32_t* coarse_lists = nullptr;
+    size_t coarse_lists_cap = 0;
     uint32_t* spill = nullptr;         // overflow list (record indices)
     size_t spill_cap = 0;
     AlphaRecord* alpha = nullptr;      // only once a draw has alpha-tested materials
@@ -107,7 +111,7 @@ struct Scratch {
 
     void release() {
         void* ptrs[] = { records, clip, visible_list, meshlet_counts, bin_counts, bin_flags, clip_overflow, bin_lists,
-                         bin_order, spill, alpha, scratch };
+                         bin_order, coarse_counts, coarse_lists, spill, alpha, scratch };
         for (void* q : ptrs)
             if (q) (void)hipFree(q);
         *this = Scratch();
@@ -724,16 +728,40 @@ void make_view(glimp_framebuffer* f, glimp_scene* s, uint32_t meshlet_offset, ui
     V.spill_keys = f->spill_keys;
 }
 
-// Lays out bins for `views` (bin_base, bins_x/y) and returns the total.
-uint32_t layout_bins(std::vector<ViewParams>& views, uint32_t bin_size) {
-    uint32_t base = 0;
+// Screen bins of a launch: all views' bins and their coarser bins.
+struct BinTotals {
+    uint32_t bins = 0, l1 = 0, l2 = 0;
+};
+
+// List capacity of a coarser bin: `times` the bin capacity, at most every
+// record slot of the launch.
+size_t coarse_capacity(size_t bin_capacity, size_t times, size_t record_slots) {
+    return std::min(bin_capacity * times, record_slots);
+}
+
+// Lays out the bins of `views` (ViewParams::bin_base to l2_x). A view gets a
+// coarser level only where a record's box can be over the finer one's limit,
+// so small views cost no coarse lists (the lists add at most half the memory
+// of the fine ones).
+BinTotals layout_bins(std::vector<ViewParams>& views, uint32_t bin_size) {
+    BinTotals t;
     for (auto& V : views) {
-        V.bin_base = base;
+        V.bin_base = t.bins;
         V.bins_x = ((uint32_t)V.width + bin_size - 1) / bin_size;
         V.bins_y = ((uint32_t)V.height + bin_size - 1) / bin_size;
-        base += V.bins_x * V.bins_y;
+        t.bins += V.bins_x * V.bins_y;
+        V.l1_base = t.l1;
+        V.l2_base = t.l2;
+        V.l1_x = V.l2_x = 0;
+        if (V.bins_x * V.bins_y <= kFinePairs) continue;
+        V.l1_x = (V.bins_x + 3) / 4;
+        const uint32_t l1_y = (V.bins_y + 3) / 4;
+        t.l1 += V.l1_x * l1_y;
+        if (V.l1_x * l1_y <= kCoarsePairs) continue;
+        V.l2_x = (V.bins_x + 15) / 16;
+        t.l2 += V.l2_x * ((V.bins_y + 15) / 16);
     }
-    return base;
+    return t;
 }
 
 // Bin indices are packed with a 6-bit lane number into 32 bits when binning.
@@ -749,8 +777,9 @@ uint64_t count_bins(const std::vector<ViewParams>& views, uint32_t bin_size) {
 // The overflow list takes each record at most once: one entry per record slot.
 size_t spill_capacity_for(size_t record_slots) { return record_slots; }
 
-int prepare_scratch(Scratch& S, size_t total_meshlets, size_t clipq, size_t total_bins, const LaunchShape& sh,
+int prepare_scratch(Scratch& S, size_t total_meshlets, size_t clipq, const BinTotals& bins, const LaunchShape& sh,
                     bool binned, bool alpha) {
+    const size_t total_bins = bins.bins;
     const size_t recs = total_meshlets * 128 + clipq * 8;
     int rc = grow_one(S.records, S.records_cap, recs);
     if (rc == GLIMP_OK) rc = grow_one(S.clip, S.clip_cap, clipq);
@@ -768,6 +797,10 @@ int prepare_scratch(Scratch& S, size_t total_meshlets, size_t clipq, size_t tota
     if (rc == GLIMP_OK && S.bin_flags_cap != old_flags_cap)
         HIP_TRY(hipMemset(S.bin_flags, 0, S.bin_flags_cap * sizeof(uint32_t)));
     if (rc == GLIMP_OK && binned) rc = grow_one(S.bin_lists, S.bin_lists_cap, total_bins * sh.bin_capacity);
+    if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_counts, S.coarse_counts_cap, (size_t)bins.l1 + bins.l2);
+    if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_lists, S.coarse_lists_cap,
+                                             bins.l1 * coarse_capacity(sh.bin_capacity, 4, recs) +
+                                                 bins.l2 * coarse_capacity(sh.bin_capacity, 16, recs));
     if (rc == GLIMP_OK && binned) rc = grow_one(S.bin_order, S.bin_order_cap, total_bins * kBinBuckets);
     if (rc == GLIMP_OK && binned) rc = grow_one(S.spill, S.spill_cap, spill_capacity_for(recs));
     if (rc == GLIMP_OK && alpha) rc = grow_one(S.alpha, S.alpha_cap, S.records_cap);
@@ -778,10 +811,10 @@ int prepare_scratch(Scratch& S, size_t total_meshlets, size_t clipq, size_t tota
     return rc;
 }
 
-void fill_params(glimp_context* c, const Scratch& S, size_t total_meshlets, size_t clipq, uint32_t total_bins,
+void fill_params(glimp_context* c, const Scratch& S, size_t total_meshlets, size_t clipq, const BinTotals& bins,
                  const LaunchShape& sh, uint32_t flags, bool alpha, DrawParams& p) {
     p.total_meshlets = (uint32_t)total_meshlets;
-    p.total_bins = total_bins;
+    p.total_bins = bins.bins;
     p.flags = flags;
     p.tables = c->approx();
     p.visible_list = S.visible_list;
@@ -803,6 +836,12 @@ void fill_params(glimp_context* c, const Scratch& S, size_t total_meshlets, size
     p.raster_threads = sh.raster_threads;
     p.bin_counts = S.bin_counts;
     p.bin_lists = S.bin_lists;
+    p.coarse_counts = S.coarse_counts;
+    p.coarse_lists = S.coarse_lists;
+    p.coarse_l1 = bins.l1;
+    p.coarse_total = bins.l1 + bins.l2;
+    p.l1_capacity = (uint32_t)coarse_capacity(sh.bin_capacity, 4, total_meshlets * 128 + clipq * 8);
+    p.l2_capacity = (uint32_t)coarse_capacity(sh.bin_capacity, 16, total_meshlets * 128 + clipq * 8);
     p.bin_order = S.bin_order;
     p.spill = S.spill;
     p.spill_capacity = (uint32_t)std::min(spill_capacity_for(total_meshlets * 128 + clipq * 8), S.spill_cap);
@@ -879,14 +918,14 @@ int glimp_draw_meshlets(glimp_context* c, glimp_framebuffer* f, glimp_scene* s, 
     std::vector<ViewParams> views(1);
     make_view(f, s, d->meshlet_offset, d->meshlet_count, d->object_to_clip, d->frustum_planes, d->flags, views[0],
               d->occlusion ? &occ : nullptr);
-    const uint32_t total_bins = direct ? 0 : layout_bins(views, sh.bin_size);
+    const BinTotals bins = direct ? BinTotals() : layout_bins(views, sh.bin_size);
     const bool alpha = (s->has_alpha && !overdraw) || deferred;    // FS_Overdraw has no alpha test
     const size_t clipq = clip_capacity_for(d->meshlet_count);
-    int rc = prepare_scratch(c->draw_scratch, d->meshlet_count, clipq, total_bins, sh, !direct, alpha);
+    int rc = prepare_scratch(c->draw_scratch, d->meshlet_count, clipq, bins, sh, !direct, alpha);
     if (rc != GLIMP_OK) return rc;
     DrawParams p;
     memset(&p, 0, sizeof(p));
-    fill_params(c, c->draw_scratch, d->meshlet_count, clipq, total_bins, sh, d->flags, alpha, p);
+    fill_params(c, c->draw_scratch, d->meshlet_count, clipq, bins, sh, d->flags, alpha, p);
     p.num_views = 1;
     p.views = nullptr;
     p.view = views[0];
@@ -982,7 +1021,7 @@ struct glimp_batch {
     ViewParams* d_views = nullptr;
     size_t total_meshlets = 0;
     size_t clip_triangles = 0;         // clip queue capacity (batch_clip_capacity)
-    uint32_t total_bins = 0;
+    BinTotals bins;
     LaunchShape shape;
     bool alpha = false;                // a view's scene has alpha-tested materials
     Scratch scratch;
@@ -1013,10 +1052,10 @@ int layout_batch(glimp_batch* b) {
     std::vector<ViewParams> probe = b->views;
     if (count_bins(probe, b->shape.bin_size) >= kMaxBins)
         return fail(GLIMP_E_LIMIT, "glimp_batch: more than 2^26 screen bins; use a larger bin size or fewer views");
-    b->total_bins = layout_bins(b->views, b->shape.bin_size);
+    b->bins = layout_bins(b->views, b->shape.bin_size);
     b->alpha = false;
     for (const auto& d : b->descs) b->alpha = b->alpha || d.scene->has_alpha;
-    int rc = prepare_scratch(b->scratch, b->total_meshlets, b->clip_triangles, b->total_bins, b->shape, true,
+    int rc = prepare_scratch(b->scratch, b->total_meshlets, b->clip_triangles, b->bins, b->shape, true,
                              b->alpha);
     if (rc != GLIMP_OK) return rc;
     if (!b->d_views) HIP_TRY(dev_alloc(&b->d_views, b->views.size()));
@@ -1027,7 +1066,7 @@ int layout_batch(glimp_batch* b) {
 
 void batch_params(glimp_batch* b, DrawParams& p) {
     memset(&p, 0, sizeof(p));
-    fill_params(b->ctx, b->scratch, b->total_meshlets, b->clip_triangles, b->total_bins, b->shape, 0, b->alpha, p);
+    fill_params(b->ctx, b->scratch, b->total_meshlets, b->clip_triangles, b->bins, b->shape, 0, b->alpha, p);
     p.num_views = (uint32_t)b->views.size();
     p.views = b->d_views;
 }

@@ -317,6 +317,7 @@ __global__ void __launch_bounds__(256) k_cull(DrawParams p) {
         p.scratch->num_clip_overflow = 0;
         p.scratch->max_bin_count = 0;
     }
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < p.coarse_total; i += gridDim.x * 256) p.coarse_counts[i] = 0;
     // the block's meshlets are consecutive: one search for the first view,
     // then each thread walks forward from it
     if (threadIdx.x == 0) s_view0 = view_of_meshlet(p, first);
@@ -1559,8 +1560,12 @@ __device__ __forceinline__ uint32_t wave_sort_u32(uint32_t v, uint32_t lane) {
 // pair counts, then their next free slots, live in LDS.
 constexpr uint32_t kRectBins = 1024;
 
+// Bins a lane walks for its own records; a wave with a larger record box
+// walks its pairs in parallel instead.
+constexpr uint32_t kWalkPairs = 16;
+
 struct BinScratch {                     // one wave's slice of the block's LDS
-    // per record: first pair, first bin, bin-box width | bins per row << 16,
+    // per record: first pair, first bin, bin-box width (| bins per row << 16),
     // record index, overflow flag (64 records a call in bin_records, 128 in
     // bin_meshlet)
     uint32_t start[128], org[128], bw[128], ridx[128], spill[128];
@@ -1569,26 +1574,63 @@ struct BinScratch {                     // one wave's slice of the block's LDS
     uint32_t slots[kRectBins];          // per rect bin: pairs, then next slot
 };
 
-// Inserts the wave's records (one per lane where `valid`) into the screen
-// bins of their views.
-__device__ void bin_records(const DrawParams& p, bool valid, const TriRecord& rec, uint32_t ridx, uint32_t lane,
-                            BinScratch& sm, unsigned long long& entries) {
-    uint32_t nb = 0, org = 0, bw = 0, pitch = 0;
+// One level's bins of a view.
+struct LevelBins {
+    uint32_t* counts;                   // the view's first bin
+    uint32_t* lists;
+    uint32_t capacity, pitch;
+};
+
+__device__ __forceinline__ LevelBins level_bins(const DrawParams& p, const ViewParams& V, uint32_t level) {
+    LevelBins L;
+    if (level == 0) {
+        L.counts = p.bin_counts + V.bin_base;
+        L.lists = p.bin_lists + (size_t)V.bin_base * p.bin_capacity;
+        L.capacity = p.bin_capacity;
+        L.pitch = V.bins_x;
+    } else if (level == 1) {
+        L.counts = p.coarse_counts + V.l1_base;
+        L.lists = p.coarse_lists + (size_t)V.l1_base * p.l1_capacity;
+        L.capacity = p.l1_capacity;
+        L.pitch = V.l1_x;
+    } else {
+        L.counts = p.coarse_counts + p.coarse_l1 + V.l2_base;
+        L.lists = p.coarse_lists + (size_t)p.coarse_l1 * p.l1_capacity + (size_t)V.l2_base * p.l2_capacity;
+        L.capacity = p.l2_capacity;
+        L.pitch = V.l2_x;
+    }
+    return L;
+}
+
+// A record with a pair past its bin's capacity goes to the overflow list
+// once and is flagged, so the bins that did take it skip it: the overflow
+// raster draws it over its whole render box.
+__device__ __forceinline__ void list_spilled(const DrawParams& p, bool spilled, uint32_t ridx, uint32_t flags,
+                                             uint32_t lane) {
+    const unsigned long long spm = __ballot(spilled);
+    if (!spm) return;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(&p.scratch->num_spill, (uint32_t)__popcll(spm));
+    base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
+    if (spilled) {
+        p.spill[base + mbcnt(spm)] = ridx;
+        p.records[ridx].flags = flags | kRecSpilled;
+    }
+}
+
+// Inserts the wave's records (one per lane where `valid`, bin boxes lo..hi,
+// x | y << 16) into one level's bins, 64 pairs at a time: for meshlets whose
+// records spread over more than kRectBins bins.
+__device__ void bin_records(const DrawParams& p, const LevelBins& L, bool valid, uint32_t lo, uint32_t hi,
+                            uint32_t flags, uint32_t ridx, uint32_t lane, BinScratch& sm) {
+    uint32_t nb = 0, org = 0, bw = 1;
     if (valid) {
-        const ViewParams& V = view_of(p, rec.flags >> 16);
-        uint32_t bmin, bmax;
-        render_bbox(rec.pos[0], rec.pos[1], rec.pos[2], V.width / 2, V.height / 2, bmin, bmax);
-        uint32_t bx0 = (uint32_t)lo16(bmin) >> p.bin_shift, by0 = (uint32_t)hi16(bmin) >> p.bin_shift;
-        uint32_t bx1 = (uint32_t)(lo16(bmax) - 1) >> p.bin_shift, by1 = (uint32_t)(hi16(bmax) - 1) >> p.bin_shift;
-        bw = bx1 - bx0 + 1;
-        nb = bw * (by1 - by0 + 1);
-        // first bin of the record's box, in the global bin numbering
-        org = V.bin_base + by0 * V.bins_x + bx0;
-        pitch = V.bins_x;
+        bw = (hi & 0xFFFFu) - (lo & 0xFFFFu) + 1;
+        nb = bw * ((hi >> 16) - (lo >> 16) + 1);
+        org = (lo >> 16) * L.pitch + (lo & 0xFFFFu);
     }
     const uint32_t incl = wave_scan_add(nb);
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-    entries += total;
     __builtin_amdgcn_wave_barrier();   // the previous call's reads of `sm` are done
     // Starts must not decrease with the lane for the search below: an
     // invalid lane (nb = 0) gets the empty range at the running total. The
@@ -1597,7 +1639,7 @@ __device__ void bin_records(const DrawParams& p, bool valid, const TriRecord& re
     // lanes after it.
     sm.start[lane] = incl - nb;
     sm.org[lane] = org;
-    sm.bw[lane] = bw | (pitch << 16);
+    sm.bw[lane] = bw;
     sm.ridx[lane] = ridx;
     sm.spill[lane] = 0;
     __builtin_amdgcn_wave_barrier();
@@ -1611,10 +1653,9 @@ __device__ void bin_records(const DrawParams& p, bool valid, const TriRecord& re
             for (uint32_t step = 32; step > 0; step >>= 1) {
                 if (sm.start[k + step] <= j) k += step;
             }
-            const uint32_t q = j - sm.start[k];
-            const uint32_t w = sm.bw[k] & 0xFFFFu, pitch_k = sm.bw[k] >> 16;
+            const uint32_t q = j - sm.start[k], w = sm.bw[k];
             const uint32_t dy = q / w, dx = q - dy * w;
-            item = ((sm.org[k] + dy * pitch_k + dx) << 6) | k;
+            item = ((sm.org[k] + dy * L.pitch + dx) << 6) | k;
         }
         // Small triangles of one meshlet share few bins: sort the wave's
         // pairs by bin so each run of equal bins takes its slots with one
@@ -1630,32 +1671,19 @@ __device__ void bin_records(const DrawParams& p, bool valid, const TriRecord& re
         const unsigned long long later = lane == 63 ? 0ull : heads & (~0ull << (lane + 1));
         const uint32_t runEnd = later ? (uint32_t)__ffsll((long long)later) - 1 : nvalid;
         uint32_t got = 0;
-        if (head) got = atomicAdd(&p.bin_counts[bin], runEnd - lane);
+        if (head) got = atomicAdd(&L.counts[bin], runEnd - lane);
         // first lane of this lane's run: highest head at or below it
         const unsigned long long upto = heads & (lane == 63 ? ~0ull : ((2ull << lane) - 1));
         const uint32_t runStart = upto ? 63u - (uint32_t)__clzll((long long)upto) : 0u;
         const uint32_t slot = __shfl(got, (int)runStart) + (lane - runStart);
         if (ok) {
             const uint32_t k = item & 63u;
-            if (slot < p.bin_capacity) p.bin_lists[(size_t)bin * p.bin_capacity + slot] = sm.ridx[k];
+            if (slot < L.capacity) L.lists[(size_t)bin * L.capacity + slot] = sm.ridx[k];
             else sm.spill[k] = 1;
         }
     }
-    // A record with a pair past its bin's capacity goes to the overflow list
-    // once and is flagged, so the bins that did take it skip it: the overflow
-    // raster draws it over its whole render box.
     __builtin_amdgcn_wave_barrier();
-    const bool spilled = valid && sm.spill[lane] != 0;
-    const unsigned long long spm = __ballot(spilled);
-    if (spm) {
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(&p.scratch->num_spill, (uint32_t)__popcll(spm));
-        base = __shfl(base, 0);
-        if (spilled) {
-            p.spill[base + mbcnt(spm)] = ridx;
-            p.records[ridx].flags = rec.flags | kRecSpilled;
-        }
-    }
+    list_spilled(p, valid && sm.spill[lane] != 0, ridx, flags, lane);
 }
 
 // Per-half minimum of two packed u16 values.
@@ -1663,9 +1691,53 @@ __device__ __forceinline__ uint32_t min_u16x2(uint32_t a, uint32_t b) {
     return min(a & 0xFFFFu, b & 0xFFFFu) | (min(a >> 16, b >> 16) << 16);
 }
 
-// Bins a lane walks for its own records; a wave with a larger record box
-// walks its pairs in parallel instead.
-constexpr uint32_t kLanePairs = 16;
+// Bins of a box lo..hi (x | y << 16).
+__device__ __forceinline__ uint32_t box_bins(uint32_t lo, uint32_t hi) {
+    return ((hi & 0xFFFFu) - (lo & 0xFFFFu) + 1) * ((hi >> 16) - (lo >> 16) + 1);
+}
+
+// Inserts records spread over a rectangle of more than kRectBins bins (a
+// large patch near the eye, a clipped triangle), each at the level that
+// keeps its pairs few: the bins of level 1 and 2 are 4x4 and 16x16 bins
+// large, and a bin's raster reads the lists of the three bins it lies in. A
+// triangle that covers a 1080p view has 8,160 pairs with 16-pixel bins, 510
+// at level 1 and 40 at level 2 (one wave inserts them 64 at a time, a round
+// trip to memory each). 1080p frame with 512 patches around the eye, 16-pixel
+// bins: scatter 401 -> 33 us, raster 86 -> 88 us, frame 315-389 -> 192 us.
+// Moving every record of more than 16 bins up costs the raster more than it
+// saves here (24-view batch: raster 164 -> 189 us): a coarse list also holds
+// records that miss the bin.
+__device__ void bin_levels(const DrawParams& p, bool valid, const TriRecord& rec, uint32_t ridx, uint32_t lane,
+                           BinScratch& sm, unsigned long long& entries) {
+    const unsigned long long vm = __ballot(valid);
+    if (!vm) return;
+    const uint32_t vflags = (uint32_t)__builtin_amdgcn_readlane((int)rec.flags, __ffsll((long long)vm) - 1);
+    const ViewParams& V = view_of(p, vflags >> 16);
+    uint32_t lo = 0, hi = 0, nb = 0, level = 0;
+    if (valid) {
+        uint32_t bmin, bmax;
+        render_bbox(rec.pos[0], rec.pos[1], rec.pos[2], V.width / 2, V.height / 2, bmin, bmax);
+        lo = ((uint32_t)lo16(bmin) >> p.bin_shift) | (((uint32_t)hi16(bmin) >> p.bin_shift) << 16);
+        hi = ((uint32_t)(lo16(bmax) - 1) >> p.bin_shift) | (((uint32_t)(hi16(bmax) - 1) >> p.bin_shift) << 16);
+        nb = box_bins(lo, hi);
+    }
+    if (counting(p)) entries += (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(nb), 63);
+    auto up = [](uint32_t v) { return (v >> 2) & 0x3FFF3FFFu; };     // both halves / 4
+    if (nb > kFinePairs && V.l1_x) {
+        lo = up(lo);
+        hi = up(hi);
+        level = 1;
+        if (box_bins(lo, hi) > kCoarsePairs && V.l2_x) {
+            lo = up(lo);
+            hi = up(hi);
+            level = 2;
+        }
+    }
+    for (uint32_t l = 0; l < 3; l++) {
+        const bool here = valid && level == l;
+        if (__ballot(here)) bin_records(p, level_bins(p, V, l), here, lo, hi, rec.flags, ridx, lane, sm);
+    }
+}
 
 // Inserts up to 128 records of one view (record k = lane + 64 h in slot h of
 // each lane) into the screen bins with one device atomic per bin they
@@ -1674,13 +1746,13 @@ constexpr uint32_t kLanePairs = 16;
 // atomicAdd; a second walk over the pairs writes them to those slots. Small
 // triangles of a meshlet share few bins, and a bin counter that every
 // overlapping wave increments once per pair run makes each later atomic on
-// it wait for the earlier ones. Rectangles of more than kRectBins bins go
-// through bin_records, 64 records at a time.
-__device__ void bin_meshlet(const DrawParams& p, const bool (&valid)[2], const TriRecord (&rec)[2],
+// it wait for the earlier ones. Returns false, with nothing done, for
+// rectangles of more than kRectBins bins (bin_levels takes those).
+__device__ bool bin_meshlet(const DrawParams& p, const bool (&valid)[2], const TriRecord (&rec)[2],
                             const uint32_t (&ridx)[2], uint32_t lane, BinScratch& sm,
                             unsigned long long& entries) {
     const unsigned long long vm0 = __ballot(valid[0]), vm1 = __ballot(valid[1]);
-    if (!(vm0 | vm1)) return;
+    if (!(vm0 | vm1)) return true;
     const int src = __ffsll((long long)(vm0 ? vm0 : vm1)) - 1;
     const uint32_t flags = (uint32_t)__builtin_amdgcn_readlane((int)(vm0 ? rec[0].flags : rec[1].flags), src);
     const ViewParams& V = view_of(p, flags >> 16);
@@ -1703,19 +1775,15 @@ __device__ void bin_meshlet(const DrawParams& p, const bool (&valid)[2], const T
     }
     rlo = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(rlo, 0xFFFFFFFFu, min_u16x2), 63);
     rhi = ~(uint32_t)__builtin_amdgcn_readlane((int)wave_scan(rhi, 0xFFFFFFFFu, min_u16x2), 63);
-    // with every record's box at most kLanePairs bins each lane walks its
+    // with every record's box at most kWalkPairs bins each lane walks its
     // own records' pairs (`steps` steps); otherwise the wave walks all pairs
     // in parallel, 64 at a time
     const uint32_t maxnb = wave_max(big);
-    const bool wide = maxnb > kLanePairs;
+    const bool wide = maxnb > kWalkPairs;
     const uint32_t steps = wide ? 0u : maxnb;
     const uint32_t rx0 = rlo & 0xFFFFu, ry0 = rlo >> 16;
     const uint32_t rw = (rhi & 0xFFFFu) - rx0 + 1, rh = (rhi >> 16) - ry0 + 1;
-    if (rw * rh > kRectBins) {
-        if (vm0) bin_records(p, valid[0], rec[0], ridx[0], lane, sm, entries);
-        if (vm1) bin_records(p, valid[1], rec[1], ridx[1], lane, sm, entries);
-        return;
-    }
+    if (rw * rh > kRectBins) return false;
     const uint32_t R = rw * rh;
     if (counting(p)) entries += (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(nb[0] + nb[1]), 63);
     uint32_t bw[2], org[2], rect[2];
@@ -1849,23 +1917,9 @@ __device__ void bin_meshlet(const DrawParams& p, const bool (&valid)[2], const T
         spill[0] = sm.spill[lane] != 0;
         spill[1] = sm.spill[64 + lane] != 0;
     }
-    // A record with a pair past its bin's capacity goes to the overflow list
-    // once and is flagged, so the bins that did take it skip it.
-    const bool s0 = valid[0] && spill[0], s1 = valid[1] && spill[1];
-    const unsigned long long m0 = __ballot(s0), m1 = __ballot(s1);
-    if (m0 | m1) {
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(&p.scratch->num_spill, (uint32_t)(__popcll(m0) + __popcll(m1)));
-        base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
-        if (s0) {
-            p.spill[base + mbcnt(m0)] = ridx[0];
-            p.records[ridx[0]].flags = rec[0].flags | kRecSpilled;
-        }
-        if (s1) {
-            p.spill[base + (uint32_t)__popcll(m0) + mbcnt(m1)] = ridx[1];
-            p.records[ridx[1]].flags = rec[1].flags | kRecSpilled;
-        }
-    }
+    list_spilled(p, valid[0] && spill[0], ridx[0], rec[0].flags, lane);
+    list_spilled(p, valid[1] && spill[1], ridx[1], rec[1].flags, lane);
+    return true;
 }
 
 // Binning of the meshlet records, then clipping of the queued triangles
@@ -1887,19 +1941,42 @@ __global__ void __launch_bounds__(256) k_bin_scatter(DrawParams p) {
     const uint32_t nvis = p.scratch->num_visible;
     const uint32_t nclip = min(p.scratch->num_clip, p.clip_capacity);
     const uint32_t q0 = waves - 1 - first;
-    // one visible meshlet's records at a time, the next one's count in flight
+    auto load = [&](uint32_t i, uint32_t cnt, bool (&valid)[2], TriRecord (&rec)[2], uint32_t (&ridx)[2]) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            ridx[h] = i * 128 + h * 64 + lane;
+            valid[h] = h * 64 + lane < cnt;
+            rec[h] = TriRecord{};
+            if (valid[h]) rec[h] = p.records[(size_t)i * 128 + h * 64 + lane];
+        }
+    };
+    // one visible meshlet's records at a time, the next one's count in
+    // flight; those of large triangles are noted and follow, 64 meshlets at
+    // a time
     while (i < nvis) {
-        const uint32_t next = i + waves;
-        TriRecord r0 = {}, r1 = {};
-        if (lane < cnt) r0 = p.records[(size_t)i * 128 + lane];
-        if (lane + 64 < cnt) r1 = p.records[(size_t)i * 128 + 64 + lane];
-        const uint32_t ncnt = next < nvis ? p.meshlet_counts[next] : 0u;
-        const bool valid[2] = { lane < cnt, lane + 64 < cnt };
-        const TriRecord rec[2] = { r0, r1 };
-        const uint32_t ridx[2] = { i * 128 + lane, i * 128 + 64 + lane };
-        bin_meshlet(p, valid, rec, ridx, lane, s_bins[wid], entries);
-        i = next;
-        cnt = ncnt;
+        const uint32_t i0 = i;
+        unsigned long long large = 0;
+        for (uint32_t k = 0; k < 64 && i < nvis; k++) {
+            const uint32_t next = i + waves;
+            bool valid[2];
+            TriRecord rec[2];
+            uint32_t ridx[2];
+            load(i, cnt, valid, rec, ridx);
+            const uint32_t ncnt = next < nvis ? p.meshlet_counts[next] : 0u;
+            if (!bin_meshlet(p, valid, rec, ridx, lane, s_bins[wid], entries)) large |= 1ull << k;
+            i = next;
+            cnt = ncnt;
+        }
+        while (large) {
+            const uint32_t m = i0 + (uint32_t)__builtin_ctzll(large) * waves;
+            large &= large - 1ull;
+            bool valid[2];
+            TriRecord rec[2];
+            uint32_t ridx[2];
+            load(m, p.meshlet_counts[m], valid, rec, ridx);
+            for (int h = 0; h < 2; h++)
+                bin_levels(p, valid[h], rec[h], ridx[h], lane, s_bins[wid], entries);
+        }
     }
     // Queued triangles go to the last waves of the grid, which have no
     // meshlet when the grid holds more waves than visible meshlets: clipping
@@ -1911,7 +1988,8 @@ __global__ void __launch_bounds__(256) k_bin_scatter(DrawParams p) {
         const bool v2[2] = { valid, false };
         const TriRecord r2[2] = { rec, rec };
         const uint32_t x2[2] = { ridx, 0 };
-        bin_meshlet(p, v2, r2, x2, lane, s_bins[wid], entries);
+        if (!bin_meshlet(p, v2, r2, x2, lane, s_bins[wid], entries))
+            bin_levels(p, valid, rec, ridx, lane, s_bins[wid], entries);
     }
     if (counting(p) && lane == 0 && entries) atomicAdd(&p.counters->bin_entries, entries);
 }
@@ -1958,7 +2036,24 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
     const uint32_t first_entry = tid < min(p.bin_capacity, kPrefetchEntries) ? list[tid] : 0u;
     const uint32_t count = p.bin_counts[bin];
     const uint32_t flagged = p.bin_flags[bin];
-    const uint32_t n = min(count, p.bin_capacity);
+    const uint32_t n0 = min(count, p.bin_capacity);
+    // the records of the coarser bins this bin lies in follow its own
+    uint32_t n1 = 0, n2 = 0;
+    const uint32_t *list1 = nullptr, *list2 = nullptr;
+    if (V.l1_x) {
+        const uint32_t c1 = V.l1_base + (by >> 2) * V.l1_x + (bx >> 2);
+        n1 = min(p.coarse_counts[c1], p.l1_capacity);
+        list1 = p.coarse_lists + (size_t)c1 * p.l1_capacity;
+        if (V.l2_x) {
+            const uint32_t c2 = V.l2_base + (by >> 4) * V.l2_x + (bx >> 4);
+            n2 = min(p.coarse_counts[p.coarse_l1 + c2], p.l2_capacity);
+            list2 = p.coarse_lists + (size_t)p.coarse_l1 * p.l1_capacity + (size_t)c2 * p.l2_capacity;
+        }
+    }
+    const uint32_t n = n0 + n1 + n2;
+    auto entry = [&](uint32_t e) {
+        return e < n0 ? list[e] : (e < n0 + n1 ? list1[e - n0] : list2[e - n0 - n1]);
+    };
     // records on the overflow list and the fan triangles of triangles that
     // found the clip queue full were drawn into the view's spill keys, which
     // flagged the bins they reached
@@ -1988,6 +2083,7 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
 
     const bool countFrags = counting(p);
     uint32_t covered = 0, passed = 0, tiles = 0;
+    bool touched = false;              // a record's box reaches the bin
     const uint32_t g = tid >> 4, px = tid & 3, py = (tid >> 2) & 3;
     constexpr bool kMasked = BS <= 32;
     constexpr uint32_t kTilesX = BS / 4;                                   // tiles per bin row
@@ -1999,13 +2095,14 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
         unsigned long long tmask = 0;      // candidate tiles of this thread's record
         BinTri<BS> t;
         if (e < n) {
-            const uint32_t r = (base == 0 && e < kPrefetchEntries) ? first_entry : list[e];
+            const uint32_t r = (e < n0 && e < kPrefetchEntries) ? first_entry : entry(e);
             const TriRecord rec = p.records[r];
             uint32_t bmin, bmax;
             TriLds f;
             load_tri(rec, hw, hh, f, bmin, bmax);
             const uint32_t cx0 = max((uint32_t)lo16(bmin), x0), cy0 = max((uint32_t)hi16(bmin), y0);
             const uint32_t cx1 = min((uint32_t)lo16(bmax), x1), cy1 = min((uint32_t)hi16(bmax), y1);
+            touched = touched || (cx1 > cx0 && cy1 > cy0);
             if constexpr (Alpha) talpha[tid] = (rec.flags & kRecAlpha) ? r : 0xFFFFFFFFu;
             t.a12 = f.a12; t.a20 = f.a20; t.a01 = f.a01;
             t.b12 = f.b12; t.b20 = f.b20; t.b01 = f.b01;
@@ -2252,7 +2349,8 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
         }
     }
     // the bin's count, read by every thread before the first barrier of the
-    // record loop (count > 0 means the loop ran), is cleared for the next draw
+    // record loop (count > 0 means the loop ran), is cleared for the next
+    // draw (the cull clears the coarser bins' counts, which 16 or 256 bins read)
     if (tid == 0 && count) p.bin_counts[bin] = 0;
     if (countFrags) {
         for (int d = 32; d > 0; d >>= 1) {
@@ -2265,7 +2363,7 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
         }
         // one lane of each 16-lane group counted the group's tiles
         if ((tid & 15u) == 0 && tiles) atomicAdd(&p.counters->tile_lanes, 16ull * tiles);
-        if (tid == 0 && n) atomicAdd(&p.counters->bins_rasterized, 1ull);
+        if (__syncthreads_or(touched) && tid == 0) atomicAdd(&p.counters->bins_rasterized, 1ull);
     }
 }
 
