@@ -797,7 +797,8 @@ int prepare_scratch(Scratch& S, size_t total_meshlets, size_t clipq, const BinTo
     if (rc == GLIMP_OK && S.bin_flags_cap != old_flags_cap)
         HIP_TRY(hipMemset(S.bin_flags, 0, S.bin_flags_cap * sizeof(uint32_t)));
     if (rc == GLIMP_OK && binned) rc = grow_one(S.bin_lists, S.bin_lists_cap, total_bins * sh.bin_capacity);
-    if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_counts, S.coarse_counts_cap, (size_t)bins.l1 + bins.l2);
+    if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_counts, S.coarse_counts_cap,
+                                             std::max<size_t>((size_t)bins.l1 + bins.l2, 1));
     if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_lists, S.coarse_lists_cap,
                                              bins.l1 * coarse_capacity(sh.bin_capacity, 4, recs) +
                                                  bins.l2 * coarse_capacity(sh.bin_capacity, 16, recs));
@@ -878,8 +879,17 @@ int glimp_draw_meshlets(glimp_context* c, glimp_framebuffer* f, glimp_scene* s, 
     HIP_TRY(hipSetDevice(c->device));
     const bool overdraw = d->pipeline == GLIMP_PIPELINE_OVERDRAW;
     const bool deferred = d->pipeline == GLIMP_PIPELINE_DEFERRED;
-    const bool direct = overdraw || deferred || (d->flags & GLIMP_DRAW_DIRECT) != 0;
+    const bool layers = overdraw || deferred;
+    const bool direct = !layers && (d->flags & GLIMP_DRAW_DIRECT) != 0;
+    if (layers) {
+        sh = LaunchShape();
+        sh.bin_size = kLayerBin;
+    }
     hipStream_t st = (hipStream_t)stream;
+    // the first draw of the pipeline since the clear starts its layers: zero
+    // counts and the clear depth, or the clear colour (layer 2 of a deferred
+    // framebuffer keeps its contents)
+    const bool first = layers && f->content != (int)d->pipeline;
     if (deferred) {
         // FS_EncodeGBuffer samples the texture of every meshlet's material
         // (Shading.cpp:357-366); without one the reference reads through a
@@ -894,19 +904,8 @@ int glimp_draw_meshlets(glimp_context* c, glimp_framebuffer* f, glimp_scene* s, 
             HIP_TRY(dev_alloc(&f->aux, 2 * n));
             HIP_TRY(hipMemsetAsync(f->aux, 0, 2 * n * 4, st));
         }
-        if (f->content != (int)GLIMP_PIPELINE_DEFERRED)   // Clear's colour; layer 2 keeps its contents
-            HIP_TRY(launch_fill32(f->aux, (uint32_t)n, f->clear_color, st));
     }
-    if (overdraw && f->content != (int)GLIMP_PIPELINE_OVERDRAW) {
-        // first overdraw draw since the clear: zero counts, depth = clear depth
-        const size_t n = (size_t)f->width * f->height;
-        if (!f->aux) HIP_TRY(dev_alloc(&f->aux, 2 * n));
-        uint32_t db;
-        memcpy(&db, &f->clear_depth, 4);
-        HIP_TRY(launch_clear(f->keys, (uint32_t)n, 0ull, st));
-        HIP_TRY(launch_fill32(f->aux, (uint32_t)n, db, st));
-        f->pending_clear = false;
-    }
+    if (overdraw && !f->aux) HIP_TRY(dev_alloc(&f->aux, 2 * (size_t)f->width * f->height));
     if (direct) HIP_TRY(flush_clear(f, st));
 
     Occlusion occ;
@@ -932,9 +931,13 @@ int glimp_draw_meshlets(glimp_context* c, glimp_framebuffer* f, glimp_scene* s, 
     p.view.aux = f->aux;
     memcpy(p.view.o2w, d->object_to_world, sizeof(p.view.o2w));
     p.deferred = deferred ? 1u : 0u;
+    p.layers = layers ? 1u : 0u;
+    p.layers_fresh = first ? 1u : 0u;
+    p.layers_clear = f->clear_color;
+    if (overdraw) p.view.fresh = first ? 1 : 0;
     // clipped triangles without queue or record room are drawn at once only by
     // the vis-buffer pipeline; the others count them in `dropped`
-    p.exact_overflow = (overdraw || deferred) ? 0u : 1u;
+    p.exact_overflow = layers ? 0u : 1u;
     if (overdraw) HIP_TRY(launch_draw_overdraw(p, st, &c->prof));
     else if (deferred) HIP_TRY(launch_draw_deferred(p, st, &c->prof));
     else if (direct) HIP_TRY(launch_draw_direct(p, st, &c->prof));

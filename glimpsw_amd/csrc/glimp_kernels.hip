@@ -18,6 +18,8 @@
 //   k_bin_raster  one workgroup per bin: LDS-resident 64-bit keys from the
 //                 bin's list, merged with its spill keys when marked
 //   k_raster_direct  without binning, all records: global 64-bit atomicMax
+//   k_bin_overdraw, k_bin_gbuffer  the overdraw and deferred pipelines' bins,
+//                 k_raster_overdraw, k_gbuffer their overflow lists
 //
 // Depth test. The reference keeps the nearest fragment (reverse-Z, strictly
 // greater depth wins, Shading.cpp:313) and, with one thread, resolves ties in
@@ -247,6 +249,8 @@ __device__ __forceinline__ uint32_t view_of_bin(const DrawParams& p, uint32_t b)
 }
 
 __device__ __forceinline__ bool counting(const DrawParams& p) { return (p.flags & 8u) != 0; }
+// The bin counters belong to the vis-buffer pipeline.
+__device__ __forceinline__ bool counting_bins(const DrawParams& p) { return counting(p) && !p.layers; }
 
 // ---------------------------------------------------------------- cull
 
@@ -1282,256 +1286,6 @@ __global__ void __launch_bounds__(256) k_raster_direct(DrawParams p) {
     }
 }
 
-// The overdraw pipeline: Rasterizer::DrawTriangle with FS_Overdraw
-// (Rasterizer.h:281-324, Shading.cpp:333-342). Every 4x4 tile of a
-// triangle's render box with a covered pixel adds one to each of its 16
-// pixels: to the covered count when the pixel is covered, else to the
-// quad-helper count; and raises each pixel's depth to the triangle's plane
-// depth there (extrapolated for uncovered pixels) when that is greater.
-// Counts and maxima commute, so the result does not depend on the order in
-// which triangles are drawn. Counts are 32-bit halves of one 64-bit word
-// per pixel (saturated to 16 bits when read); the depth maximum is a 32-bit
-// max on the float's bits, taken only for positive depths, which order like
-// their bits (the stored depth starts at the clear depth, >= +0).
-__global__ void __launch_bounds__(256) k_raster_overdraw(DrawParams p) {
-    __shared__ TriLds tl[4][64];
-    __shared__ uint32_t tview[4][64];
-    const uint32_t wid = threadIdx.x / kWave;
-    const uint32_t lane = lane_id();
-    const uint32_t nchunks = num_chunks(p);
-    const bool countFrags = counting(p);
-    const uint32_t waves = gridDim.x * 4;
-    const unsigned long long groupMask = 0xFFFFull << (lane & 48u);
-
-    for (uint32_t c = blockIdx.x * 4 + wid; c < nchunks; c += waves) {
-        const Chunk ck = get_chunk(p, c);
-        if (ck.count == 0) continue;
-        uint32_t ntiles = 0;
-        TriLds t;
-        if (lane < ck.count) {
-            const uint32_t r = ck.list ? ck.list[ck.base + lane] : ck.base + lane;
-            const TriRecord rec = p.records[r];
-            const uint32_t v = rec.flags >> 16;
-            const ViewParams& V = view_of(p, v);
-            uint32_t bmin, bmax;
-            load_tri(rec, V.width / 2, V.height / 2, t, bmin, bmax);
-            t.org = bmin;
-            const uint32_t tw = (uint32_t)(lo16(bmax) - lo16(bmin)) >> 2;
-            const uint32_t th = (uint32_t)(hi16(bmax) - hi16(bmin)) >> 2;
-            t.tw = tw;
-            ntiles = tw * th;
-            tview[wid][lane] = v;
-        }
-        const uint32_t incl = wave_scan_add(ntiles);
-        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-        t.start = incl - ntiles;
-        if (lane < ck.count) tl[wid][lane] = t;
-        else tl[wid][lane].start = 0xFFFFFFFFu;
-        __builtin_amdgcn_wave_barrier();
-
-        uint32_t covered = 0;
-        const uint32_t sub = lane >> 4, px = lane & 3, py = (lane >> 2) & 3;
-        for (uint32_t base = 0; base < total; base += 4) {
-            const uint32_t j = base + sub;
-            bool cov = false, inside = false;
-            float depth = 0.0f;
-            uint32_t off = 0;
-            unsigned long long* keys = nullptr;
-            uint32_t* dbuf = nullptr;
-            if (j < total) {
-                uint32_t k = 0;
-#pragma unroll
-                for (uint32_t step = 32; step > 0; step >>= 1) {
-                    if (tl[wid][k + step].start <= j) k += step;
-                }
-                const TriLds& T = tl[wid][k];
-                const ViewParams& V = view_of(p, tview[wid][k]);
-                const uint32_t W = (uint32_t)V.width;
-                const uint32_t pt = j - T.start;
-                const uint32_t ty = pt / T.tw;
-                const uint32_t tx = pt - ty * T.tw;
-                const uint32_t x = (uint32_t)lo16(T.org) + tx * 4 + px;
-                const uint32_t y = (uint32_t)hi16(T.org) + ty * 4 + py;
-                const int32_t w0 = edge_at(T.e0, T.a12, T.b12, x, y);
-                const int32_t w1 = edge_at(T.e1, T.a20, T.b20, x, y);
-                const int32_t w2 = edge_at(T.e2, T.a01, T.b01, x, y);
-                // render boxes lie inside the framebuffer; the bounds test
-                // only guards the stores
-                inside = x < W && y < (uint32_t)V.height;
-                cov = inside && (w0 | w1 | w2) >= 0;
-                depth = __builtin_fmaf((float)w1, T.z10, __builtin_fmaf((float)w2, T.z20, T.z0));
-                off = pixel_offset(W, x, y);
-                keys = V.keys;
-                dbuf = V.aux;
-            }
-            if (!(__ballot(cov) & groupMask) || !inside) continue;
-            atomicAdd(keys + off, cov ? (1ull << 32) : 1ull);
-            if (depth > 0.0f) {
-                const uint32_t bits = fbits(depth);
-                if (bits > __atomic_load_n(dbuf + off, __ATOMIC_RELAXED)) atomicMax(dbuf + off, bits);
-            }
-            covered += cov ? 1u : 0u;
-        }
-        if (countFrags) {
-            for (int d = 32; d > 0; d >>= 1) covered += __shfl_xor(covered, d);
-            if (lane == 0) {
-                atomicAdd(&p.counters->fragments_covered, (unsigned long long)covered);
-                atomicAdd(&p.counters->fragments_passed, (unsigned long long)covered);
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-
-// cvttps2udq: truncation; NaN and results outside [0, 2^32) give 0xFFFFFFFF.
-__device__ __forceinline__ uint32_t cvt_trunc_u32(float x) {
-    if (!(x > -1.0f && x < 4294967296.0f)) return 0xFFFFFFFFu;
-    return (uint32_t)x;
-}
-
-// The layer-2 word of FS_EncodeGBuffer (Shading.cpp:397-401): MapOctahedron
-// (Texture.h:282-288) of the remapped normal, each coordinate as
-// conv<uint32_t>(oct * 1023 + 0.5) in 10 bits, then the NMR texel's
-// metallic and roughness bytes cut to 6 bits. The optimised build folds
-// (c * 0.5 + 0.5) * 1023 + 0.5 into fma(c, 511.5, 512), sums the absolute
-// values left to right, takes 1/sum from VRCP14PS alone and evaluates
-// max(-z * w, 0) as zero unless positive.
-__device__ __forceinline__ uint32_t gbuffer_pack(const ApproxTables& T, const float n[3], uint32_t nmr) {
-    const float w = rcp14(T, (fabsf(n[0]) + fabsf(n[1])) + fabsf(n[2]));
-    const float mz = -n[2] * w;
-    const float t = mz > 0.0f ? mz : 0.0f;
-    const float u = __builtin_fmaf(n[0], w, mulsign(t, n[0]));
-    const float v = __builtin_fmaf(n[1], w, mulsign(t, n[1]));
-    uint32_t r = cvt_trunc_u32(__builtin_fmaf(u, 511.5f, 512.0f));
-    r |= cvt_trunc_u32(__builtin_fmaf(v, 511.5f, 512.0f)) << 10;
-    r |= ((nmr >> 18) & 0x3Fu) << 20;
-    r |= ((nmr >> 26) & 0x3Fu) << 26;
-    return r;
-}
-
-// FS_EncodeGBuffer's attribute stores (Shading.cpp:357-401) as a second pass
-// over the draw's records, after the vis-buffer raster has settled which
-// fragment wins each pixel (depth test, draw order and the alpha test,
-// which FS_EncodeGBuffer applies to every material). A fragment wins when
-// its key equals the pixel's final key; keys are unique per fragment, so
-// exactly one fragment per covered pixel writes, and the result is the
-// reference's last write. A tile with a winning fragment computes UVs and
-// levels on all 16 lanes (derivatives and the filter choice span the tile),
-// samples the base colour and, for two-layer textures, the NMR texel, and
-// the winning lanes write the colour and the packed normal / metallic /
-// roughness word (zero for one-layer textures). Meshlets of a deferred
-// draw all have textured materials (checked on the host), so every record
-// has its alpha record.
-__global__ void __launch_bounds__(256) k_gbuffer(DrawParams p) {
-    __shared__ TriLds tl[4][64];
-    __shared__ uint32_t tview[4][64];
-    __shared__ uint32_t talpha[4][64];
-    const uint32_t wid = threadIdx.x / kWave;
-    const uint32_t lane = lane_id();
-    const uint32_t nchunks = num_chunks(p);
-    const uint32_t waves = gridDim.x * 4;
-    const unsigned long long groupMask = 0xFFFFull << (lane & 48u);
-    const ApproxTables& AT = p.tables;
-
-    for (uint32_t c = blockIdx.x * 4 + wid; c < nchunks; c += waves) {
-        const Chunk ck = get_chunk(p, c);
-        if (ck.count == 0) continue;
-        uint32_t ntiles = 0;
-        TriLds t;
-        if (lane < ck.count) {
-            const uint32_t r = ck.list ? ck.list[ck.base + lane] : ck.base + lane;
-            const TriRecord rec = p.records[r];
-            const uint32_t v = rec.flags >> 16;
-            const ViewParams& V = view_of(p, v);
-            uint32_t bmin, bmax;
-            load_tri(rec, V.width / 2, V.height / 2, t, bmin, bmax);
-            t.org = bmin;
-            const uint32_t tw = (uint32_t)(lo16(bmax) - lo16(bmin)) >> 2;
-            const uint32_t th = (uint32_t)(hi16(bmax) - hi16(bmin)) >> 2;
-            t.tw = tw;
-            ntiles = tw * th;
-            tview[wid][lane] = v;
-            talpha[wid][lane] = (rec.flags & kRecAlpha) ? r : 0xFFFFFFFFu;
-        }
-        const uint32_t incl = wave_scan_add(ntiles);
-        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-        t.start = incl - ntiles;
-        if (lane < ck.count) tl[wid][lane] = t;
-        else tl[wid][lane].start = 0xFFFFFFFFu;
-        __builtin_amdgcn_wave_barrier();
-
-        const uint32_t sub = lane >> 4, px = lane & 3, py = (lane >> 2) & 3;
-        for (uint32_t base = 0; base < total; base += 4) {
-            const uint32_t j = base + sub;
-            bool match = false;
-            uint32_t k = 0, off = 0;
-            int32_t w1 = 0, w2 = 0;
-            if (j < total) {
-#pragma unroll
-                for (uint32_t step = 32; step > 0; step >>= 1) {
-                    if (tl[wid][k + step].start <= j) k += step;
-                }
-                const TriLds& T = tl[wid][k];
-                const ViewParams& V = view_of(p, tview[wid][k]);
-                const uint32_t W = (uint32_t)V.width;
-                const uint32_t pt = j - T.start;
-                const uint32_t ty = pt / T.tw;
-                const uint32_t tx = pt - ty * T.tw;
-                const uint32_t x = (uint32_t)lo16(T.org) + tx * 4 + px;
-                const uint32_t y = (uint32_t)hi16(T.org) + ty * 4 + py;
-                const int32_t w0 = edge_at(T.e0, T.a12, T.b12, x, y);
-                w1 = edge_at(T.e1, T.a20, T.b20, x, y);
-                w2 = edge_at(T.e2, T.a01, T.b01, x, y);
-                const float depth = __builtin_fmaf((float)w1, T.z10, __builtin_fmaf((float)w2, T.z20, T.z0));
-                if (x < W && y < (uint32_t)V.height && (w0 | w1 | w2) >= 0 && depth > V.clear_depth) {
-                    off = pixel_offset(W, x, y);
-                    const unsigned long long key = ((unsigned long long)fbits(depth) << 32) | T.keylo;
-                    match = V.keys[off] == key;
-                }
-            }
-            // uniform per 16-lane group: the group shares j, hence the record
-            if (!(__ballot(match) & groupMask)) continue;
-            const uint32_t ai = talpha[wid][k];
-            if (ai == 0xFFFFFFFFu) continue;
-            const TriLds& T = tl[wid][k];
-            const ViewParams& V = view_of(p, tview[wid][k]);
-            const AlphaRecord& A = p.alpha[ai];
-            const DevTexture& tex = V.textures[A.tex & 0xFFFFFFu];
-            const TileUV uv = tile_uv(AT, A, ((T.keylo >> 7) & 1u) == 0, tex, w1, w2, lane);
-            const uint32_t baseColor = sample_level(tex, uv.U, uv.V, uv.mip, !uv.minify);
-            uint32_t ch2 = 0;
-            if (tex.num_layers >= 2) {
-                const uint32_t nmr = sample_level(tex, uv.U, uv.V, uv.mip, !uv.minify, 1);
-                if (match) {
-                    // the fragment's triangle: meshlet and primitive from its rank
-                    const uint32_t rank = ~T.keylo;
-                    const uint32_t prim = ((rank >> 8) & 7u) * 16u + ((rank >> 3) & 15u);
-                    const uint32_t mi = V.meshlet_offset + ((rank >> 11) - V.seq_base);
-                    const uint8_t* I = V.m.indices + (size_t)mi * 384;
-                    float nv[3][3], tv[3][3];
-#pragma unroll
-                    for (int q = 0; q < 3; q++) {
-                        const uint32_t nt = V.m.normal_tangents[(size_t)mi * 64 + (I[q * 128 + prim] & 63u)];
-                        unpack_normal(AT, nt, nv[q]);
-                        unpack_normal(AT, nt >> 16, tv[q]);
-                    }
-                    const uint32_t handed = (uint32_t)((V.m.tangent_handedness[mi] >> (I[prim] & 63u)) & 1u) << 31;
-                    float N[3], Tw[3];
-                    lerp_to_world(AT, nv, uv.b, V.o2w, N);
-                    lerp_to_world(AT, tv, uv.b, V.o2w, Tw);
-                    normal_map(AT, N, Tw, handed, nmr);
-                    ch2 = gbuffer_pack(AT, N, nmr);
-                }
-            }
-            if (match) {
-                V.aux[off] = baseColor;
-                V.aux[(size_t)V.width * V.height + off] = ch2;
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-}
-
 // ---------------------------------------------------------------- binning
 
 constexpr uint32_t kSortedBinningPairs = 128;
@@ -1703,7 +1457,7 @@ __device__ __forceinline__ uint32_t box_bins(uint32_t lo, uint32_t hi) {
 // triangle that covers a 1080p view has 8,160 pairs with 16-pixel bins, 510
 // at level 1 and 40 at level 2 (one wave inserts them 64 at a time, a round
 // trip to memory each). 1080p frame with 512 patches around the eye, 16-pixel
-// bins: scatter 401 -> 33 us, raster 86 -> 88 us, frame 315-389 -> 192 us.
+// bins: scatter 401 -> 33 us, raster 86 -> 89 us, frame 296 -> 177 us.
 // Moving every record of more than 16 bins up costs the raster more than it
 // saves here (24-view batch: raster 164 -> 189 us): a coarse list also holds
 // records that miss the bin.
@@ -1991,7 +1745,80 @@ __global__ void __launch_bounds__(256) k_bin_scatter(DrawParams p) {
         if (!bin_meshlet(p, v2, r2, x2, lane, s_bins[wid], entries))
             bin_levels(p, valid, rec, ridx, lane, s_bins[wid], entries);
     }
-    if (counting(p) && lane == 0 && entries) atomicAdd(&p.counters->bin_entries, entries);
+    if (counting_bins(p) && lane == 0 && entries) atomicAdd(&p.counters->bin_entries, entries);
+}
+
+// The 4x4 tiles of a box of tw x th tiles that a triangle can cover, bit ty *
+// kTilesX + tx, from its edge steps and its edge values W0 at the box's
+// first pixel, one tile row at a time. Each edge's largest value over a
+// tile's 16 pixels is V = D + 4A tx + 4B ty, D = e + max(0, 3A) + max(0, 3B)
+// at the box's first tile; a tile where one V is negative has no covered
+// pixel. Along a row V >= 0 holds on one side of q = -(D + 4B ty) / 4A: tx
+// >= q for A > 0, tx <= q for A < 0. q comes from a float reciprocal
+// (relative error a few 2^-24, far below the 2^-10 margin taken outward over
+// the |q| <= 16 that matter), so the mask keeps every tile with a covered
+// pixel. Edge values inside a render box stay below 2^31 in magnitude (|e| <
+// 2^27, |A|, |B| < 2^17, pixel coordinates below 2^12), so D + 4B ty is exact.
+template <uint32_t kTilesX>
+__device__ __forceinline__ unsigned long long tile_mask(const int32_t (&A)[3], const int32_t (&Bv)[3],
+                                                        const int32_t (&W0)[3], uint32_t tw, uint32_t th) {
+    unsigned long long mask = 0;
+    if (!tw) return mask;
+    int32_t D[3];
+    float nr[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        D[i] = W0[i] + max(0, 3 * A[i]) + max(0, 3 * Bv[i]);
+        nr[i] = A[i] != 0 ? -__builtin_amdgcn_rcpf((float)(4 * A[i])) : 0.0f;
+    }
+    for (uint32_t ty = 0; ty < th; ty++) {
+        int32_t lo = 0, hi = (int32_t)tw - 1;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const int32_t R = D[i] + __mul24(Bv[i], (int32_t)(4 * ty));
+            const float q = fminf(fmaxf((float)R * nr[i], -16.0f), 16.0f);
+            if (A[i] > 0) lo = max(lo, (int32_t)ceilf(q - 0x1p-10f));
+            else if (A[i] < 0) hi = min(hi, (int32_t)floorf(q + 0x1p-10f));
+            else if (R < 0) hi = -1;
+        }
+        if (hi >= lo) mask |= (unsigned long long)((2u << hi) - (1u << lo)) << (ty * kTilesX);
+    }
+    return mask;
+}
+
+// The lists of records whose box may reach a bin: its own, and those of the
+// coarser bins it lies in. Wave-uniform.
+struct BinLists {
+    const uint32_t *fine, *l1, *l2;
+    uint32_t n0, n1, n2;
+    uint32_t count0;               // the bin's own count, with pairs past its capacity
+
+    __device__ __forceinline__ uint32_t count() const { return n0 + n1 + n2; }
+    __device__ __forceinline__ uint32_t operator[](uint32_t e) const {
+        return e < n0 ? fine[e] : (e < n0 + n1 ? l1[e - n0] : l2[e - n0 - n1]);
+    }
+};
+
+__device__ __forceinline__ BinLists bin_lists(const DrawParams& p, const ViewParams& V, uint32_t bin, uint32_t bx,
+                                              uint32_t by) {
+    // the three counts are loaded side by side (a level the view lacks reads
+    // the first count): one round trip to memory instead of three in a row
+    const uint32_t c1 = V.l1_x ? V.l1_base + (by >> 2) * V.l1_x + (bx >> 2) : 0u;
+    const uint32_t c2 = V.l2_x ? V.l2_base + (by >> 4) * V.l2_x + (bx >> 4) : 0u;
+    uint32_t k0 = p.bin_counts[bin], k1 = p.coarse_counts[c1];
+    uint32_t k2 = p.coarse_counts[V.l2_x ? p.coarse_l1 + c2 : 0u];
+    k0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)k0);
+    k1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)k1);
+    k2 = (uint32_t)__builtin_amdgcn_readfirstlane((int)k2);
+    BinLists l;
+    l.count0 = k0;
+    l.fine = p.bin_lists + (size_t)bin * p.bin_capacity;
+    l.n0 = min(k0, p.bin_capacity);
+    l.l1 = p.coarse_lists + (size_t)c1 * p.l1_capacity;
+    l.n1 = V.l1_x ? min(k1, p.l1_capacity) : 0u;
+    l.l2 = p.coarse_lists + (size_t)p.coarse_l1 * p.l1_capacity + (size_t)c2 * p.l2_capacity;
+    l.n2 = V.l2_x ? min(k2, p.l2_capacity) : 0u;
+    return l;
 }
 
 // One block per bin of any view. The bin's keys live in LDS in the same 4x4
@@ -2034,26 +1861,9 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
     constexpr uint32_t kPrefetchEntries = kThreads < 128 ? kThreads : 128;
     const uint32_t* list = p.bin_lists + (size_t)bin * p.bin_capacity;
     const uint32_t first_entry = tid < min(p.bin_capacity, kPrefetchEntries) ? list[tid] : 0u;
-    const uint32_t count = p.bin_counts[bin];
     const uint32_t flagged = p.bin_flags[bin];
-    const uint32_t n0 = min(count, p.bin_capacity);
-    // the records of the coarser bins this bin lies in follow its own
-    uint32_t n1 = 0, n2 = 0;
-    const uint32_t *list1 = nullptr, *list2 = nullptr;
-    if (V.l1_x) {
-        const uint32_t c1 = V.l1_base + (by >> 2) * V.l1_x + (bx >> 2);
-        n1 = min(p.coarse_counts[c1], p.l1_capacity);
-        list1 = p.coarse_lists + (size_t)c1 * p.l1_capacity;
-        if (V.l2_x) {
-            const uint32_t c2 = V.l2_base + (by >> 4) * V.l2_x + (bx >> 4);
-            n2 = min(p.coarse_counts[p.coarse_l1 + c2], p.l2_capacity);
-            list2 = p.coarse_lists + (size_t)p.coarse_l1 * p.l1_capacity + (size_t)c2 * p.l2_capacity;
-        }
-    }
-    const uint32_t n = n0 + n1 + n2;
-    auto entry = [&](uint32_t e) {
-        return e < n0 ? list[e] : (e < n0 + n1 ? list1[e - n0] : list2[e - n0 - n1]);
-    };
+    const BinLists lists = bin_lists(p, V, bin, bx, by);
+    const uint32_t n = lists.count(), count = lists.count0;
     // records on the overflow list and the fan triangles of triangles that
     // found the clip queue full were drawn into the view's spill keys, which
     // flagged the bins they reached
@@ -2095,14 +1905,19 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
         unsigned long long tmask = 0;      // candidate tiles of this thread's record
         BinTri<BS> t;
         if (e < n) {
-            const uint32_t r = (e < n0 && e < kPrefetchEntries) ? first_entry : entry(e);
+            uint32_t r = first_entry;
+            if (base + kThreads <= lists.n0) {          // nearly always: a chunk of the bin's own list
+                if (base || e >= kPrefetchEntries) r = lists.fine[e];
+            } else if (e >= min(lists.n0, kPrefetchEntries)) {
+                r = lists[e];
+            }
             const TriRecord rec = p.records[r];
             uint32_t bmin, bmax;
             TriLds f;
             load_tri(rec, hw, hh, f, bmin, bmax);
             const uint32_t cx0 = max((uint32_t)lo16(bmin), x0), cy0 = max((uint32_t)hi16(bmin), y0);
             const uint32_t cx1 = min((uint32_t)lo16(bmax), x1), cy1 = min((uint32_t)hi16(bmax), y1);
-            touched = touched || (cx1 > cx0 && cy1 > cy0);
+            if (countFrags) touched = touched || (cx1 > cx0 && cy1 > cy0);
             if constexpr (Alpha) talpha[tid] = (rec.flags & kRecAlpha) ? r : 0xFFFFFFFFu;
             t.a12 = f.a12; t.a20 = f.a20; t.a01 = f.a01;
             t.b12 = f.b12; t.b20 = f.b20; t.b01 = f.b01;
@@ -2125,43 +1940,9 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
                 t.li0 = ((cx0 - x0) << 2) + (cy0 - y0) * BS;
             }
             if constexpr (kMasked) {
-                // The tiles of the box that the triangle can cover, one tile
-                // row at a time. Each edge's largest value over a tile's 16
-                // pixels is V = D + 4A tx + 4B ty, D = e + max(0, 3A) +
-                // max(0, 3B) at the box's first tile; a tile where one V is
-                // negative has no covered pixel. Along a row V >= 0 holds on
-                // one side of q = -(D + 4B ty) / 4A: tx >= q for A > 0, tx <= q
-                // for A < 0. q comes from a float reciprocal (relative error a
-                // few 2^-24, far below the 2^-10 margin taken outward over the
-                // |q| <= 16 that matter), so the mask keeps every tile with a
-                // covered pixel. Edge values inside a render box stay below 2^31
-                // in magnitude (|e| < 2^27, |A|, |B| < 2^17, pixel coordinates
-                // below 2^12), so D + 4B ty is exact.
-                unsigned long long mask = 0;
-                if (tw) {
-                    const int32_t A[3] = {f.a12, f.a20, f.a01}, Bv[3] = {f.b12, f.b20, f.b01};
-                    const int32_t W0[3] = {t.w0, t.w1, t.w2};
-                    int32_t D[3];
-                    float nr[3];
-#pragma unroll
-                    for (int i = 0; i < 3; i++) {
-                        D[i] = W0[i] + max(0, 3 * A[i]) + max(0, 3 * Bv[i]);
-                        nr[i] = A[i] != 0 ? -__builtin_amdgcn_rcpf((float)(4 * A[i])) : 0.0f;
-                    }
-                    for (uint32_t ty = 0; ty < th; ty++) {
-                        int32_t lo = 0, hi = (int32_t)tw - 1;
-#pragma unroll
-                        for (int i = 0; i < 3; i++) {
-                            const int32_t R = D[i] + __mul24(Bv[i], (int32_t)(4 * ty));
-                            const float q = fminf(fmaxf((float)R * nr[i], -16.0f), 16.0f);
-                            if (A[i] > 0) lo = max(lo, (int32_t)ceilf(q - 0x1p-10f));
-                            else if (A[i] < 0) hi = min(hi, (int32_t)floorf(q + 0x1p-10f));
-                            else if (R < 0) hi = -1;
-                        }
-                        if (hi >= lo)
-                            mask |= (unsigned long long)((2u << hi) - (1u << lo)) << (ty * kTilesX);
-                    }
-                }
+                const int32_t A[3] = {f.a12, f.a20, f.a01}, Bv[3] = {f.b12, f.b20, f.b01};
+                const int32_t W0[3] = {t.w0, t.w1, t.w2};
+                const unsigned long long mask = tile_mask<kTilesX>(A, Bv, W0, tw, th);
                 tmask = mask;
                 ntiles = (uint32_t)__popcll(mask);
             } else {
@@ -2351,7 +2132,8 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
     // the bin's count, read by every thread before the first barrier of the
     // record loop (count > 0 means the loop ran), is cleared for the next
     // draw (the cull clears the coarser bins' counts, which 16 or 256 bins read)
-    if (tid == 0 && count) p.bin_counts[bin] = 0;
+    // (a deferred draw's G-buffer pass still reads it)
+    if (tid == 0 && count && !(Alpha && p.layers)) p.bin_counts[bin] = 0;
     if (countFrags) {
         for (int d = 32; d > 0; d >>= 1) {
             covered += __shfl_xor(covered, d);
@@ -2362,8 +2144,13 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
             atomicAdd(&p.counters->fragments_passed, (unsigned long long)passed);
         }
         // one lane of each 16-lane group counted the group's tiles
-        if ((tid & 15u) == 0 && tiles) atomicAdd(&p.counters->tile_lanes, 16ull * tiles);
-        if (__syncthreads_or(touched) && tid == 0) atomicAdd(&p.counters->bins_rasterized, 1ull);
+        if ((tid & 15u) == 0 && tiles && counting_bins(p)) atomicAdd(&p.counters->tile_lanes, 16ull * tiles);
+        const unsigned long long tm = __ballot(touched);
+        if (lane == 0) s_wave_total[wid] = tm ? 1u : 0u;
+        __syncthreads();
+        uint32_t any = 0;
+        for (uint32_t w = 0; w < (uint32_t)kWaves; w++) any |= s_wave_total[w];
+        if (any && tid == 0 && counting_bins(p)) atomicAdd(&p.counters->bins_rasterized, 1ull);
     }
 }
 
@@ -2431,6 +2218,27 @@ __global__ void __launch_bounds__(256) k_bin_order(DrawParams p) {
     if (valid) p.bin_order[(size_t)cls * p.total_bins + s_base[cls] + rank] = bin;
 }
 
+// The bin at a position of the heavy-first order: every class size in one
+// load, then the class holding the position without branches (a search that
+// stops at the first class large enough loads the sizes one after another).
+__device__ __forceinline__ uint32_t ordered_bin(const DrawParams& p, uint32_t item) {
+    uint32_t n[kBinBuckets];
+#pragma unroll
+    for (uint32_t c = 0; c < kBinBuckets; c++) n[c] = p.scratch->bucket[c];
+    uint32_t cls = 0, start = 0, acc = 0;
+    bool found = false;
+#pragma unroll
+    for (int c = (int)kBinBuckets - 1; c >= 0; c--) {
+        const bool here = !found && item - acc < n[c];
+        cls = here ? (uint32_t)c : cls;
+        start = here ? acc : start;
+        found = found || here;
+        acc += n[c];
+    }
+    // (every position is in a class)
+    return found ? p.bin_order[(size_t)cls * p.total_bins + (item - start)] : item;
+}
+
 // One block per bin; block i rasterizes the i-th bin of the heavy-first
 // order, so the blocks dispatched first (the hardware starts blocks in
 // index order) get the crowded bins. (Taking the position from a ticket
@@ -2444,29 +2252,523 @@ __global__ void __launch_bounds__(kThreads) k_bin_raster(DrawParams p) {
     __shared__ uint32_t s_wave_total[kThreads / kWave];
     __shared__ uint32_t talpha[Alpha ? kThreads : 1];
     __shared__ uint32_t s_bin;
-    if (threadIdx.x == 0) {
-        // every class size in one load, then the class holding position
-        // blockIdx.x without branches (a search that stops at the first
-        // class large enough loads the sizes one after another)
-        uint32_t n[kBinBuckets];
-#pragma unroll
-        for (uint32_t c = 0; c < kBinBuckets; c++) n[c] = p.scratch->bucket[c];
-        const uint32_t item = blockIdx.x;
-        uint32_t cls = 0, start = 0, acc = 0;
-        bool found = false;
-#pragma unroll
-        for (int c = (int)kBinBuckets - 1; c >= 0; c--) {
-            const bool here = !found && item - acc < n[c];
-            cls = here ? (uint32_t)c : cls;
-            start = here ? acc : start;
-            found = found || here;
-            acc += n[c];
-        }
-        // (every position is in a class)
-        s_bin = found ? p.bin_order[(size_t)cls * p.total_bins + (item - start)] : item;
-    }
+    if (threadIdx.x == 0) s_bin = ordered_bin(p, blockIdx.x);
     __syncthreads();
-    raster_bin<BS, kThreads, Alpha>(p, s_bin, keys, tl, tmasks, s_wave_total, talpha);
+    // wave-uniform: the bin's corners, its view and list addresses are scalars
+    raster_bin<BS, kThreads, Alpha>(p, (uint32_t)__builtin_amdgcn_readfirstlane((int)s_bin), keys, tl, tmasks, s_wave_total, talpha);
+}
+
+// ---------------------------------------------------------------- layer pipelines
+
+// A block's walk over a bin's records for the pipelines that keep more than
+// a key per pixel: the records' candidate tiles split evenly over the 16-lane
+// groups as in raster_bin. visit(T, record, w0, w1, w2, li) is called by the
+// 16 lanes of a tile together, li being the lane's pixel in the bin's
+// 4x4-tiled order. Records on the overflow list are left to the pipeline's
+// overflow pass.
+template <int BS, int kThreads>
+struct BinWalk {
+    BinTriMask tl[kThreads];
+    unsigned long long masks[kThreads];
+    uint32_t record[kThreads];
+    uint32_t wave_total[kThreads / kWave];
+};
+
+template <int BS, int kThreads, class Visit>
+__device__ __forceinline__ void walk_bin(const DrawParams& p, const ViewParams& V, const BinLists& lists, uint32_t x0,
+                                         uint32_t y0, uint32_t x1, uint32_t y1, BinWalk<BS, kThreads>& sm,
+                                         Visit visit) {
+    static_assert(BS <= 32, "a bin's tiles are one 64-bit mask");
+    constexpr uint32_t kGroups = kThreads / 16, kTilesX = BS / 4;
+    constexpr uint32_t kTileShift = kTilesX == 2 ? 1u : (kTilesX == 4 ? 2u : 3u);
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
+    const uint32_t g = tid >> 4, px = tid & 3, py = (tid >> 2) & 3;
+    const int hw = V.width / 2, hh = V.height / 2;
+    const uint32_t n = lists.count();
+    for (uint32_t base = 0; base < n; base += kThreads) {
+        const uint32_t e = base + tid;
+        unsigned long long mask = 0;
+        BinTriMask t = {};
+        if (e < n) {
+            const uint32_t r = lists[e];
+            const TriRecord rec = p.records[r];
+            uint32_t bmin, bmax;
+            TriLds f;
+            load_tri(rec, hw, hh, f, bmin, bmax);
+            const uint32_t cx0 = max((uint32_t)lo16(bmin), x0), cy0 = max((uint32_t)hi16(bmin), y0);
+            const uint32_t cx1 = min((uint32_t)lo16(bmax), x1), cy1 = min((uint32_t)hi16(bmax), y1);
+            if (cx1 > cx0 && cy1 > cy0 && !(rec.flags & kRecSpilled)) {
+                t.a12 = f.a12; t.a20 = f.a20; t.a01 = f.a01;
+                t.b12 = f.b12; t.b20 = f.b20; t.b01 = f.b01;
+                t.z0 = f.z0; t.z10 = f.z10; t.z20 = f.z20;
+                t.keylo = f.keylo;
+                t.w0 = edge_at(f.e0, f.a12, f.b12, cx0, cy0);
+                t.w1 = edge_at(f.e1, f.a20, f.b20, cx0, cy0);
+                t.w2 = edge_at(f.e2, f.a01, f.b01, cx0, cy0);
+                t.li0 = ((cx0 - x0) << 2) + (cy0 - y0) * BS;
+                const int32_t A[3] = { f.a12, f.a20, f.a01 }, B[3] = { f.b12, f.b20, f.b01 };
+                const int32_t W0[3] = { t.w0, t.w1, t.w2 };
+                mask = tile_mask<kTilesX>(A, B, W0, (cx1 - cx0) >> 2, (cy1 - cy0) >> 2);
+                sm.record[tid] = r;
+            }
+        }
+        const uint32_t ntiles = (uint32_t)__popcll(mask);
+        const uint32_t incl = wave_scan_add(ntiles);
+        if (lane == 63) sm.wave_total[wid] = incl;
+        __syncthreads();
+        uint32_t prev = 0, total = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < (uint32_t)(kThreads / kWave); w++) {
+            const uint32_t val = sm.wave_total[w];
+            if (w < wid) prev += val;
+            total += val;
+        }
+        t.start = e < n ? prev + incl - ntiles : 0xFFFFFFFFu;
+        sm.tl[tid] = t;
+        sm.masks[tid] = mask;
+        __syncthreads();
+        const uint32_t per = (total + kGroups - 1) / kGroups;
+        uint32_t j = min(g * per, total);
+        const uint32_t j1 = min(j + per, total);
+        if (j < j1) {
+            uint32_t k = 0;
+#pragma unroll
+            for (uint32_t step = kThreads / 2; step > 0; step >>= 1)
+                if (sm.tl[k + step].start <= j) k += step;
+            BinTriMask T = sm.tl[k];
+            unsigned long long m = sm.masks[k];
+            for (uint32_t skip = j - T.start; skip; skip--) m &= m - 1ull;
+            for (;;) {
+                const uint32_t b = (uint32_t)__builtin_ctzll(m);
+                m &= m - 1ull;
+                const uint32_t tx = b & (kTilesX - 1), ty = b >> kTileShift;
+                const int32_t mx = (int32_t)(px + 4 * tx), my = (int32_t)(py + 4 * ty);
+                visit(T, k, (int32_t)((uint32_t)T.w0 + (uint32_t)__mul24(T.a12, mx) + (uint32_t)__mul24(T.b12, my)),
+                      (int32_t)((uint32_t)T.w1 + (uint32_t)__mul24(T.a20, mx) + (uint32_t)__mul24(T.b20, my)),
+                      (int32_t)((uint32_t)T.w2 + (uint32_t)__mul24(T.a01, mx) + (uint32_t)__mul24(T.b01, my)),
+                      T.li0 + (tx << 4) + ty * (4 * BS) + px + (py << 2));
+                if (++j >= j1) break;
+                if (!m) {          // tiles remain in the range: a later record has them
+                    do {
+                        m = sm.masks[++k];
+                    } while (!m);
+                    T = sm.tl[k];
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// A block's bin of the (single) view of a layer pipeline's draw.
+struct LayerBin {
+    uint32_t bin, x0, y0, x1, y1, bx, by;
+};
+
+__device__ __forceinline__ LayerBin layer_bin(const DrawParams& p, const ViewParams& V, uint32_t bin, uint32_t size) {
+    LayerBin b;
+    b.bin = bin;
+    b.by = (bin - V.bin_base) / V.bins_x;
+    b.bx = (bin - V.bin_base) - b.by * V.bins_x;
+    b.x0 = b.bx * size;
+    b.y0 = b.by * size;
+    b.x1 = min(b.x0 + size, (uint32_t)V.width);
+    b.y1 = min(b.y0 + size, (uint32_t)V.height);
+    return b;
+}
+
+// Element i of a bin's 4x4-tiled pixels in the framebuffer's order; false
+// past the framebuffer's edge.
+template <int BS>
+__device__ __forceinline__ bool bin_element(const ViewParams& V, const LayerBin& b, uint32_t i, size_t& at) {
+    const uint32_t strip = i / (BS * 4), rem = i % (BS * 4);
+    at = (size_t)(b.y0 + strip * 4) * (uint32_t)V.width + b.x0 * 4 + rem;
+    return rem < (b.x1 - b.x0) * 4 && b.y0 + strip * 4 < b.y1;
+}
+
+// Records of the overflow list, 64 a wave (record index = list[base + i]).
+__device__ __forceinline__ uint32_t spill_chunks(const DrawParams& p) {
+    return (min(p.scratch->num_spill, p.spill_capacity) + 63) / 64;
+}
+
+__device__ __forceinline__ Chunk spill_chunk(const DrawParams& p, uint32_t c) {
+    Chunk k;
+    k.base = c * 64;
+    k.count = min(64u, min(p.scratch->num_spill, p.spill_capacity) - c * 64);
+    k.list = p.spill;
+    return k;
+}
+
+// The overdraw pipeline: Rasterizer::DrawTriangle with FS_Overdraw
+// (Rasterizer.h:281-324, Shading.cpp:333-342). Every 4x4 tile of a
+// triangle's render box with a covered pixel adds one to each of its 16
+// pixels: to the covered count when the pixel is covered, else to the
+// quad-helper count; and raises each pixel's depth to the triangle's plane
+// depth there (extrapolated for uncovered pixels) when that is greater.
+// Counts and maxima commute, so the result does not depend on the order in
+// which triangles are drawn. Counts are 32-bit halves of one 64-bit word
+// per pixel (saturated to 16 bits when read); the depth maximum is a 32-bit
+// max on the float's bits, taken only for positive depths, which order like
+// their bits (the stored depth starts at the clear depth, >= +0).
+//
+// One block per bin counts in LDS and writes the bin once. 1600x900, eight
+// layers, 350,000 records (27 M tile lanes): 66 us, bound by the tile walk
+// like the bin raster; with a 64-bit and a 32-bit global atomic per tile and
+// pixel and 64 records a wave it took 647 us.
+template <int BS, int kThreads>
+__global__ void __launch_bounds__(kThreads) k_bin_overdraw(DrawParams p) {
+    __shared__ BinWalk<BS, kThreads> sm;
+    __shared__ uint32_t counts[2][BS * BS];    // covered, helper
+    __shared__ uint32_t depths[BS * BS];
+    __shared__ uint32_t s_bin;
+    if (threadIdx.x == 0) s_bin = ordered_bin(p, blockIdx.x);
+    __syncthreads();
+    const ViewParams& V = p.view;
+    const LayerBin b = layer_bin(p, V, s_bin, BS);
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    const unsigned long long groupMask = 0xFFFFull << (lane & 48u);
+    const BinLists lists = bin_lists(p, V, b.bin, b.bx, b.by);
+    const uint32_t count = lists.count0;
+    if (b.bin == 0 && tid == 0) p.scratch->num_visible = 0;    // its last reader is done
+    if (lists.count() == 0 && !V.fresh) return;
+    for (uint32_t i = tid; i < BS * BS; i += kThreads) {
+        size_t at;
+        const bool in = bin_element<BS>(V, b, i, at);
+        counts[0][i] = counts[1][i] = 0;
+        depths[i] = (V.fresh || !in) ? fbits(V.clear_depth) : V.aux[at];
+    }
+    uint32_t covered = 0;
+    walk_bin<BS, kThreads>(p, V, lists, b.x0, b.y0, b.x1, b.y1, sm,
+                           [&](const BinTriMask& T, uint32_t, int32_t w0, int32_t w1, int32_t w2, uint32_t li) {
+        const bool cov = (w0 | w1 | w2) >= 0;
+        if (!(__ballot(cov) & groupMask)) return;
+        const float depth = __builtin_fmaf((float)w1, T.z10, __builtin_fmaf((float)w2, T.z20, T.z0));
+        atomicAdd(&counts[cov ? 0 : 1][li], 1u);
+        if (depth > 0.0f) atomicMax(&depths[li], fbits(depth));
+        covered += cov ? 1u : 0u;
+    });
+    __syncthreads();
+    for (uint32_t i = tid; i < BS * BS; i += kThreads) {
+        size_t at;
+        if (!bin_element<BS>(V, b, i, at)) continue;
+        const unsigned long long old = V.fresh ? 0ull : V.keys[at];
+        V.keys[at] = old + (((unsigned long long)counts[0][i] << 32) + counts[1][i]);
+        V.aux[at] = depths[i];
+    }
+    if (tid == 0 && count) p.bin_counts[b.bin] = 0;
+    if (counting(p)) {
+        for (int d = 32; d > 0; d >>= 1) covered += __shfl_xor(covered, d);
+        if (lane == 0) {
+            atomicAdd(&p.counters->fragments_covered, (unsigned long long)covered);
+            atomicAdd(&p.counters->fragments_passed, (unsigned long long)covered);
+        }
+    }
+}
+
+// The same for the records of the overflow list, after the bins, with global
+// atomics.
+__global__ void __launch_bounds__(256) k_raster_overdraw(DrawParams p) {
+    __shared__ TriLds tl[4][64];
+    __shared__ uint32_t tview[4][64];
+    const uint32_t wid = threadIdx.x / kWave;
+    const uint32_t lane = lane_id();
+    const uint32_t nchunks = spill_chunks(p);
+    const bool countFrags = counting(p);
+    const uint32_t waves = gridDim.x * 4;
+    const unsigned long long groupMask = 0xFFFFull << (lane & 48u);
+
+    for (uint32_t c = blockIdx.x * 4 + wid; c < nchunks; c += waves) {
+        const Chunk ck = spill_chunk(p, c);
+        uint32_t ntiles = 0;
+        TriLds t;
+        if (lane < ck.count) {
+            const uint32_t r = ck.list[ck.base + lane];
+            const TriRecord rec = p.records[r];
+            const uint32_t v = rec.flags >> 16;
+            const ViewParams& V = view_of(p, v);
+            uint32_t bmin, bmax;
+            load_tri(rec, V.width / 2, V.height / 2, t, bmin, bmax);
+            t.org = bmin;
+            const uint32_t tw = (uint32_t)(lo16(bmax) - lo16(bmin)) >> 2;
+            const uint32_t th = (uint32_t)(hi16(bmax) - hi16(bmin)) >> 2;
+            t.tw = tw;
+            ntiles = tw * th;
+            tview[wid][lane] = v;
+        }
+        const uint32_t incl = wave_scan_add(ntiles);
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        t.start = incl - ntiles;
+        if (lane < ck.count) tl[wid][lane] = t;
+        else tl[wid][lane].start = 0xFFFFFFFFu;
+        __builtin_amdgcn_wave_barrier();
+
+        uint32_t covered = 0;
+        const uint32_t sub = lane >> 4, px = lane & 3, py = (lane >> 2) & 3;
+        for (uint32_t base = 0; base < total; base += 4) {
+            const uint32_t j = base + sub;
+            bool cov = false, inside = false;
+            float depth = 0.0f;
+            uint32_t off = 0;
+            unsigned long long* keys = nullptr;
+            uint32_t* dbuf = nullptr;
+            if (j < total) {
+                uint32_t k = 0;
+#pragma unroll
+                for (uint32_t step = 32; step > 0; step >>= 1) {
+                    if (tl[wid][k + step].start <= j) k += step;
+                }
+                const TriLds& T = tl[wid][k];
+                const ViewParams& V = view_of(p, tview[wid][k]);
+                const uint32_t W = (uint32_t)V.width;
+                const uint32_t pt = j - T.start;
+                const uint32_t ty = pt / T.tw;
+                const uint32_t tx = pt - ty * T.tw;
+                const uint32_t x = (uint32_t)lo16(T.org) + tx * 4 + px;
+                const uint32_t y = (uint32_t)hi16(T.org) + ty * 4 + py;
+                const int32_t w0 = edge_at(T.e0, T.a12, T.b12, x, y);
+                const int32_t w1 = edge_at(T.e1, T.a20, T.b20, x, y);
+                const int32_t w2 = edge_at(T.e2, T.a01, T.b01, x, y);
+                // render boxes lie inside the framebuffer; the bounds test
+                // only guards the stores
+                inside = x < W && y < (uint32_t)V.height;
+                cov = inside && (w0 | w1 | w2) >= 0;
+                depth = __builtin_fmaf((float)w1, T.z10, __builtin_fmaf((float)w2, T.z20, T.z0));
+                off = pixel_offset(W, x, y);
+                keys = V.keys;
+                dbuf = V.aux;
+            }
+            if (!(__ballot(cov) & groupMask) || !inside) continue;
+            atomicAdd(keys + off, cov ? (1ull << 32) : 1ull);
+            if (depth > 0.0f) {
+                const uint32_t bits = fbits(depth);
+                if (bits > __atomic_load_n(dbuf + off, __ATOMIC_RELAXED)) atomicMax(dbuf + off, bits);
+            }
+            covered += cov ? 1u : 0u;
+        }
+        if (countFrags) {
+            for (int d = 32; d > 0; d >>= 1) covered += __shfl_xor(covered, d);
+            if (lane == 0) {
+                atomicAdd(&p.counters->fragments_covered, (unsigned long long)covered);
+                atomicAdd(&p.counters->fragments_passed, (unsigned long long)covered);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// cvttps2udq: truncation; NaN and results outside [0, 2^32) give 0xFFFFFFFF.
+__device__ __forceinline__ uint32_t cvt_trunc_u32(float x) {
+    if (!(x > -1.0f && x < 4294967296.0f)) return 0xFFFFFFFFu;
+    return (uint32_t)x;
+}
+
+// The layer-2 word of FS_EncodeGBuffer (Shading.cpp:397-401): MapOctahedron
+// (Texture.h:282-288) of the remapped normal, each coordinate as
+// conv<uint32_t>(oct * 1023 + 0.5) in 10 bits, then the NMR texel's
+// metallic and roughness bytes cut to 6 bits. The optimised build folds
+// (c * 0.5 + 0.5) * 1023 + 0.5 into fma(c, 511.5, 512), sums the absolute
+// values left to right, takes 1/sum from VRCP14PS alone and evaluates
+// max(-z * w, 0) as zero unless positive.
+__device__ __forceinline__ uint32_t gbuffer_pack(const ApproxTables& T, const float n[3], uint32_t nmr) {
+    const float w = rcp14(T, (fabsf(n[0]) + fabsf(n[1])) + fabsf(n[2]));
+    const float mz = -n[2] * w;
+    const float t = mz > 0.0f ? mz : 0.0f;
+    const float u = __builtin_fmaf(n[0], w, mulsign(t, n[0]));
+    const float v = __builtin_fmaf(n[1], w, mulsign(t, n[1]));
+    uint32_t r = cvt_trunc_u32(__builtin_fmaf(u, 511.5f, 512.0f));
+    r |= cvt_trunc_u32(__builtin_fmaf(v, 511.5f, 512.0f)) << 10;
+    r |= ((nmr >> 18) & 0x3Fu) << 20;
+    r |= ((nmr >> 26) & 0x3Fu) << 26;
+    return r;
+}
+
+// Base colour and layer-2 word of the fragments of one tile of record `ai`
+// (all 16 lanes call it: derivatives and the filter choice span the tile;
+// `match` lanes get theirs).
+__device__ __forceinline__ void gbuffer_fragment(const DrawParams& p, const ViewParams& V, uint32_t ai,
+                                                 uint32_t keylo, int32_t w1, int32_t w2, bool match, uint32_t lane,
+                                                 uint32_t& color, uint32_t& ch2) {
+    const ApproxTables& AT = p.tables;
+    const AlphaRecord& A = p.alpha[ai];
+    const DevTexture& tex = V.textures[A.tex & 0xFFFFFFu];
+    const TileUV uv = tile_uv(AT, A, ((keylo >> 7) & 1u) == 0, tex, w1, w2, lane);
+    color = sample_level(tex, uv.U, uv.V, uv.mip, !uv.minify);
+    ch2 = 0;
+    if (tex.num_layers < 2) return;
+    const uint32_t nmr = sample_level(tex, uv.U, uv.V, uv.mip, !uv.minify, 1);
+    if (!match) return;
+    // the fragment's triangle: meshlet and primitive from its rank
+    const uint32_t rank = ~keylo;
+    const uint32_t prim = ((rank >> 8) & 7u) * 16u + ((rank >> 3) & 15u);
+    const uint32_t mi = V.meshlet_offset + ((rank >> 11) - V.seq_base);
+    const uint8_t* I = V.m.indices + (size_t)mi * 384;
+    float nv[3][3], tv[3][3];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const uint32_t nt = V.m.normal_tangents[(size_t)mi * 64 + (I[q * 128 + prim] & 63u)];
+        unpack_normal(AT, nt, nv[q]);
+        unpack_normal(AT, nt >> 16, tv[q]);
+    }
+    const uint32_t handed = (uint32_t)((V.m.tangent_handedness[mi] >> (I[prim] & 63u)) & 1u) << 31;
+    float N[3], Tw[3];
+    lerp_to_world(AT, nv, uv.b, V.o2w, N);
+    lerp_to_world(AT, tv, uv.b, V.o2w, Tw);
+    normal_map(AT, N, Tw, handed, nmr);
+    ch2 = gbuffer_pack(AT, N, nmr);
+}
+
+// FS_EncodeGBuffer's attribute stores (Shading.cpp:357-401) as a second pass
+// over the draw's records, after the vis-buffer raster has settled which
+// fragment wins each pixel (depth test, draw order and the alpha test,
+// which FS_EncodeGBuffer applies to every material). A fragment wins when
+// its key equals the pixel's final key; keys are unique per fragment, so
+// exactly one fragment per covered pixel writes, and the result is the
+// reference's last write. A tile with a winning fragment computes UVs and
+// levels on all 16 lanes (derivatives and the filter choice span the tile),
+// samples the base colour and, for two-layer textures, the NMR texel, and
+// the winning lanes write the colour and the packed normal / metallic /
+// roughness word (zero for one-layer textures). Meshlets of a deferred
+// draw all have textured materials (checked on the host), so every record
+// has its alpha record.
+//
+// One block per bin walks the bin's records again: 960x540, 36,600 records of
+// which some cover much of the view, 76 us beside a 43 us bin raster. Waves
+// of 64 records each, walking all their tiles with global atomics and then
+// again for the G-buffer, took 1,477 and 2,297 us: a view-sized triangle was
+// one wave's work. After a clear the pass also writes the clear colour where
+// nothing was drawn.
+template <int BS, int kThreads>
+__global__ void __launch_bounds__(kThreads) k_bin_gbuffer(DrawParams p) {
+    __shared__ BinWalk<BS, kThreads> sm;
+    __shared__ unsigned long long keys[BS * BS];
+    __shared__ uint32_t color[BS * BS], layer2[BS * BS];
+    __shared__ uint8_t won[BS * BS];
+    __shared__ uint32_t s_bin;
+    if (threadIdx.x == 0) s_bin = ordered_bin(p, blockIdx.x);
+    __syncthreads();
+    const ViewParams& V = p.view;
+    const LayerBin b = layer_bin(p, V, s_bin, BS);
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    const unsigned long long groupMask = 0xFFFFull << (lane & 48u);
+    const BinLists lists = bin_lists(p, V, b.bin, b.bx, b.by);
+    const uint32_t count = lists.count0;
+    if (lists.count() == 0 && !p.layers_fresh) return;
+    for (uint32_t i = tid; i < BS * BS; i += kThreads) {
+        size_t at;
+        const bool in = bin_element<BS>(V, b, i, at);
+        keys[i] = in ? V.keys[at] : 0ull;
+        won[i] = 0;
+    }
+    const float clearDepth = V.clear_depth;
+    walk_bin<BS, kThreads>(p, V, lists, b.x0, b.y0, b.x1, b.y1, sm,
+                           [&](const BinTriMask& T, uint32_t k, int32_t w0, int32_t w1, int32_t w2, uint32_t li) {
+        const float depth = __builtin_fmaf((float)w1, T.z10, __builtin_fmaf((float)w2, T.z20, T.z0));
+        const bool match = (w0 | w1 | w2) >= 0 && depth > clearDepth &&
+                           keys[li] == (((unsigned long long)fbits(depth) << 32) | T.keylo);
+        if (!(__ballot(match) & groupMask)) return;
+        uint32_t c, ch2;
+        gbuffer_fragment(p, V, sm.record[k], T.keylo, w1, w2, match, lane, c, ch2);
+        if (match) {
+            color[li] = c;
+            layer2[li] = ch2;
+            won[li] = 1;
+        }
+    });
+    __syncthreads();
+    const size_t pixels = (size_t)V.width * V.height;
+    for (uint32_t i = tid; i < BS * BS; i += kThreads) {
+        size_t at;
+        if (!bin_element<BS>(V, b, i, at)) continue;
+        if (won[i]) {
+            V.aux[at] = color[i];
+            V.aux[pixels + at] = layer2[i];
+        } else if (p.layers_fresh) {
+            V.aux[at] = p.layers_clear;
+        }
+    }
+    if (tid == 0 && count) p.bin_counts[b.bin] = 0;
+}
+
+// The same for the records of the overflow list, after the bins.
+__global__ void __launch_bounds__(256) k_gbuffer(DrawParams p) {
+    __shared__ TriLds tl[4][64];
+    __shared__ uint32_t tview[4][64];
+    __shared__ uint32_t talpha[4][64];
+    const uint32_t wid = threadIdx.x / kWave;
+    const uint32_t lane = lane_id();
+    const uint32_t nchunks = spill_chunks(p);
+    const uint32_t waves = gridDim.x * 4;
+    const unsigned long long groupMask = 0xFFFFull << (lane & 48u);
+
+    for (uint32_t c = blockIdx.x * 4 + wid; c < nchunks; c += waves) {
+        const Chunk ck = spill_chunk(p, c);
+        uint32_t ntiles = 0;
+        TriLds t;
+        if (lane < ck.count) {
+            const uint32_t r = ck.list[ck.base + lane];
+            const TriRecord rec = p.records[r];
+            const uint32_t v = rec.flags >> 16;
+            const ViewParams& V = view_of(p, v);
+            uint32_t bmin, bmax;
+            load_tri(rec, V.width / 2, V.height / 2, t, bmin, bmax);
+            t.org = bmin;
+            const uint32_t tw = (uint32_t)(lo16(bmax) - lo16(bmin)) >> 2;
+            const uint32_t th = (uint32_t)(hi16(bmax) - hi16(bmin)) >> 2;
+            t.tw = tw;
+            ntiles = tw * th;
+            tview[wid][lane] = v;
+            talpha[wid][lane] = (rec.flags & kRecAlpha) ? r : 0xFFFFFFFFu;
+        }
+        const uint32_t incl = wave_scan_add(ntiles);
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        t.start = incl - ntiles;
+        if (lane < ck.count) tl[wid][lane] = t;
+        else tl[wid][lane].start = 0xFFFFFFFFu;
+        __builtin_amdgcn_wave_barrier();
+
+        const uint32_t sub = lane >> 4, px = lane & 3, py = (lane >> 2) & 3;
+        for (uint32_t base = 0; base < total; base += 4) {
+            const uint32_t j = base + sub;
+            bool match = false;
+            uint32_t k = 0, off = 0;
+            int32_t w1 = 0, w2 = 0;
+            if (j < total) {
+#pragma unroll
+                for (uint32_t step = 32; step > 0; step >>= 1) {
+                    if (tl[wid][k + step].start <= j) k += step;
+                }
+                const TriLds& T = tl[wid][k];
+                const ViewParams& V = view_of(p, tview[wid][k]);
+                const uint32_t W = (uint32_t)V.width;
+                const uint32_t pt = j - T.start;
+                const uint32_t ty = pt / T.tw;
+                const uint32_t tx = pt - ty * T.tw;
+                const uint32_t x = (uint32_t)lo16(T.org) + tx * 4 + px;
+                const uint32_t y = (uint32_t)hi16(T.org) + ty * 4 + py;
+                const int32_t w0 = edge_at(T.e0, T.a12, T.b12, x, y);
+                w1 = edge_at(T.e1, T.a20, T.b20, x, y);
+                w2 = edge_at(T.e2, T.a01, T.b01, x, y);
+                const float depth = __builtin_fmaf((float)w1, T.z10, __builtin_fmaf((float)w2, T.z20, T.z0));
+                if (x < W && y < (uint32_t)V.height && (w0 | w1 | w2) >= 0 && depth > V.clear_depth) {
+                    off = pixel_offset(W, x, y);
+                    const unsigned long long key = ((unsigned long long)fbits(depth) << 32) | T.keylo;
+                    match = V.keys[off] == key;
+                }
+            }
+            // uniform per 16-lane group: the group shares j, hence the record
+            if (!(__ballot(match) & groupMask)) continue;
+            const uint32_t ai = talpha[wid][k];
+            if (ai == 0xFFFFFFFFu) continue;
+            const ViewParams& V = view_of(p, tview[wid][k]);
+            uint32_t color, ch2;
+            gbuffer_fragment(p, V, ai, tl[wid][k].keylo, w1, w2, match, lane, color, ch2);
+            if (match) {
+                V.aux[off] = color;
+                V.aux[(size_t)V.width * V.height + off] = ch2;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
 }
 
 // Clears every scratch counter: at the end of a direct draw (the binned
@@ -2628,6 +2930,27 @@ void launch_front(const DrawParams& p, hipStream_t s, Profiler* prof, bool separ
     }
 }
 
+// Cull to ordered bins. `overflow`: the overflow list is drawn into the
+// views' spill keys.
+void launch_binning(const DrawParams& p, hipStream_t s, Profiler* prof, bool overflow) {
+    launch_front(p, s, prof, false);   // the scatter kernel clips
+    {
+        // about one chunk per wave: two per meshlet plus room for clipped records
+        const uint32_t want = max((2 * p.total_meshlets + 3) / 4 + 16, 64u);
+        if (p.alpha)
+            launch_kernel(prof, "bin_scatter", k_bin_scatter<true>,
+                          dim3(min(want, resident_blocks<k_bin_scatter<true>, 256>())), dim3(256), 0, s, p);
+        else
+            launch_kernel(prof, "bin_scatter", k_bin_scatter<false>,
+                          dim3(min(want, resident_blocks<k_bin_scatter<false>, 256>())), dim3(256), 0, s, p);
+    }
+    {
+        const dim3 grid((p.total_bins + 255) / 256 + (overflow ? kOverflowBlocks : 0u));
+        if (p.alpha) launch_kernel(prof, "bin_order", k_bin_order<true>, grid, dim3(256), 0, s, p);
+        else launch_kernel(prof, "bin_order", k_bin_order<false>, grid, dim3(256), 0, s, p);
+    }
+}
+
 }  // namespace
 
 void warm_launch_shapes() {
@@ -2635,8 +2958,6 @@ void warm_launch_shapes() {
     (void)resident_blocks<k_mesh_setup<true>, 256>();
     (void)resident_blocks<k_raster_direct<false>, 256>();
     (void)resident_blocks<k_raster_direct<true>, 256>();
-    (void)resident_blocks<k_raster_overdraw, 256>();
-    (void)resident_blocks<k_gbuffer, 256>();
     (void)resident_blocks<k_bin_scatter<false>, 256>();
     (void)resident_blocks<k_bin_scatter<true>, 256>();
 }
@@ -2667,23 +2988,17 @@ hipError_t launch_decode_overdraw(const unsigned long long* counts, const uint32
 }
 
 hipError_t launch_draw_overdraw(const DrawParams& p, hipStream_t s, Profiler* prof) {
-    launch_front(p, s, prof, true);
-    {
-        const uint32_t want = max((2 * p.total_meshlets + 3) / 4 + 16, 64u);
-        launch_kernel(prof, "raster_overdraw", k_raster_overdraw,
-                      dim3(min(want, resident_blocks<k_raster_overdraw, 256>())), dim3(256), 0, s, p);
-    }
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, s, p.scratch);
+    launch_binning(p, s, prof, false);
+    launch_kernel(prof, "bin_overdraw", k_bin_overdraw<kLayerBin, 256>, dim3(p.total_bins), dim3(256), 0, s, p);
+    launch_kernel(prof, "raster_overdraw", k_raster_overdraw, dim3(kOverflowBlocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
 hipError_t launch_draw_deferred(const DrawParams& p, hipStream_t s, Profiler* prof) {
-    launch_front(p, s, prof, true);
-    const uint32_t want = max((2 * p.total_meshlets + 3) / 4 + 16, 64u);
-    launch_kernel(prof, "raster_direct", k_raster_direct<true>,
-                  dim3(min(want, resident_blocks<k_raster_direct<true>, 256>())), dim3(256), 0, s, p);
-    launch_kernel(prof, "gbuffer", k_gbuffer, dim3(min(want, resident_blocks<k_gbuffer, 256>())), dim3(256), 0, s, p);
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, s, p.scratch);
+    hipError_t e = launch_draw_binned(p, s, prof);
+    if (e != hipSuccess) return e;
+    launch_kernel(prof, "bin_gbuffer", k_bin_gbuffer<kLayerBin, 256>, dim3(p.total_bins), dim3(256), 0, s, p);
+    launch_kernel(prof, "gbuffer", k_gbuffer, dim3(kOverflowBlocks), dim3(256), 0, s, p);
     return hipGetLastError();
 }
 
@@ -2741,22 +3056,7 @@ hipError_t launch_draw_direct(const DrawParams& p, hipStream_t s, Profiler* prof
 }
 
 hipError_t launch_draw_binned(const DrawParams& p, hipStream_t s, Profiler* prof) {
-    launch_front(p, s, prof, false);   // the scatter kernel clips
-    {
-        // about one chunk per wave: two per meshlet plus room for clipped records
-        const uint32_t want = max((2 * p.total_meshlets + 3) / 4 + 16, 64u);
-        if (p.alpha)
-            launch_kernel(prof, "bin_scatter", k_bin_scatter<true>,
-                          dim3(min(want, resident_blocks<k_bin_scatter<true>, 256>())), dim3(256), 0, s, p);
-        else
-            launch_kernel(prof, "bin_scatter", k_bin_scatter<false>,
-                          dim3(min(want, resident_blocks<k_bin_scatter<false>, 256>())), dim3(256), 0, s, p);
-    }
-    {
-        const dim3 grid((p.total_bins + 255) / 256 + kOverflowBlocks);
-        if (p.alpha) launch_kernel(prof, "bin_order", k_bin_order<true>, grid, dim3(256), 0, s, p);
-        else launch_kernel(prof, "bin_order", k_bin_order<false>, grid, dim3(256), 0, s, p);
-    }
+    launch_binning(p, s, prof, true);
     // records of alpha-tested materials need the variant with the alpha test
     if (p.alpha) {
         if (!launch_bin_raster<true>(p, s, prof)) return hipErrorInvalidValue;

@@ -124,10 +124,13 @@ struct Counters {                  // device counters, u64 each
 
 constexpr uint32_t kBinBuckets = 16;
 
+// Bin side of the overdraw and deferred pipelines.
+constexpr uint32_t kLayerBin = 16;
+
 // Bins a record's box may cover before it moves to the coarser bins, in
 // meshlets that spread over too many bins to count them in LDS, and level-1
 // bins before it moves to level 2.
-constexpr uint32_t kFinePairs = 16;
+constexpr uint32_t kFinePairs = 64;
 constexpr uint32_t kCoarsePairs = 64;
 
 // Per-draw scratch counters, cleared without a launch of their own:
@@ -221,6 +224,9 @@ struct DrawParams {
     TriRecord* records;            // [total_meshlets * 128 + clip_record_capacity]
     AlphaRecord* alpha;            // same indexing as records; null when no view has alpha-tested materials
     uint32_t deferred;             // FS_EncodeGBuffer: every textured material runs the alpha test
+    uint32_t layers;               // the overdraw or the deferred pipeline
+    uint32_t layers_fresh;         // deferred: the colour layer starts from layers_clear
+    uint32_t layers_clear;
     uint32_t* meshlet_counts;      // [total_meshlets] records kept per meshlet
     uint32_t clip_record_base;     // = total_meshlets * 128
     uint32_t clip_record_capacity;

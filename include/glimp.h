@@ -148,12 +148,14 @@ int glimp_framebuffer_keys(glimp_framebuffer* fb, void** keys, size_t* bytes);
                                        * octahedral normal (2 x 10 bits) and the metallic / roughness bytes
                                        * cut to 6 bits; a clear leaves layer 2 alone. Every drawn meshlet
                                        * needs a material with a texture (GLIMP_E_UNSUPPORTED otherwise).
-                                       * Always rasterized with per-fragment atomics (GLIMP_DRAW_DIRECT). */
+                                       * Always rasterized in 16-pixel bins (bin_size, bin_capacity and
+                                       * GLIMP_DRAW_DIRECT are ignored). */
 #define GLIMP_PIPELINE_OVERDRAW 2u    /* ShadingContext::OverdrawShader: FS_Overdraw (Shading.cpp:333-342, 656).
                                        * Layer 0 holds per pixel the covered count (high 16 bits) and the
                                        * quad-helper count (low 16 bits) added to the clear colour
                                        * (saturating), layer 1 the maximum plane depth of the tiles drawn.
-                                       * Always rasterized with per-fragment atomics (GLIMP_DRAW_DIRECT). */
+                                       * Always rasterized in 16-pixel bins (bin_size, bin_capacity and
+                                       * GLIMP_DRAW_DIRECT are ignored). */
 
 typedef struct glimp_draw_desc {
     uint32_t meshlet_offset;           /* ShadingContext::MeshletOffset */
