@@ -1742,15 +1742,23 @@ int diff_setup(glimp_context* c, glimp_scene* sc, const glimp_diff_desc* d, cons
     if (rc != GLIMP_OK) return rc;
     if (count == 0 || !views) return fail(GLIMP_E_INVALID, who + ": no views");
     std::vector<DiffView> table(count);
-    uint64_t base = 0;
+    uint64_t base = 0, blocks = 0;
     for (uint32_t i = 0; i < count; i++) {
         rc = diff_view(views[i].framebuffer, views[i].object_to_clip, (uint32_t)base, s, who, table[i]);
         if (rc != GLIMP_OK) return rc;
         base += (uint64_t)table[i].width * (uint64_t)table[i].height;
+        table[i].block_base = (uint32_t)blocks;
+        table[i].blocks_x = ((uint32_t)table[i].width + 15) / 16;
+        table[i].blocks_y = ((uint32_t)table[i].height + 15) / 16;
+        table[i].cell_w = (table[i].blocks_x + 15) / 16;
+        table[i].cell_h = (table[i].blocks_y + 15) / 16;
+        p.cell_blocks = std::max(p.cell_blocks, table[i].cell_w * table[i].cell_h);
+        blocks += (uint64_t)table[i].blocks_x * table[i].blocks_y;
         if (base >= (1ull << 31)) return fail(GLIMP_E_LIMIT, who + ": more than 2^31 pixels in one call");
     }
     p.num_views = count;
     p.total_pixels = (uint32_t)base;
+    p.total_blocks = (uint32_t)blocks;
     if (count == 1) {
         p.view = table[0];
         p.views = nullptr;
@@ -1788,8 +1796,8 @@ int diff_backward(glimp_context* c, glimp_scene* sc, const glimp_diff_desc* d, c
     if (!grad_out || !grad_texels || !grad_uv || !grad_color)
         return fail(GLIMP_E_INVALID, who + ": NULL gradient array");
     p.grad_out = (const float4*)grad_out;
-    HIP_TRY(diff_workspace_reserve(c->diff_ws, p.total_pixels));
-    HIP_TRY(launch_diff_backward(p, c->diff_ws, d->num_texels, (uint32_t)nv, (float4*)grad_texels, (float2*)grad_uv,
+    HIP_TRY(diff_workspace_reserve(c->diff_ws, p.total_pixels, p.total_blocks, sc->m.count, count));
+    HIP_TRY(launch_diff_backward(p, c->diff_ws, d->num_texels, (float4*)grad_texels, (float2*)grad_uv,
                                  (float4*)grad_color, s, &c->prof));
     return GLIMP_OK;
 }

@@ -24,6 +24,8 @@ struct DiffView {
     const DrawEntry* draws;
     uint32_t num_draws;
     uint32_t pixel_base;
+    uint32_t block_base, blocks_x, blocks_y;   // 16x16-pixel blocks of the backward, all views' in one numbering
+    uint32_t cell_w, cell_h;       // blocks per cell of the 16x16 grid over the view
     float object_to_clip[16];
     float scale_x, scale_y, center_x, center_y, kx, ky;
 };
@@ -44,39 +46,57 @@ struct DiffParams {
     const float4* color;           // [meshlets * 64]
     float4* out;                   // forward: [total_pixels]
     const float4* grad_out;        // backward: [total_pixels]
-    // backward records, 4 texel and 3 vertex records per pixel slot
+    // backward (diff.hip): a texel record per pixel slot ...
     uint32_t* tex_keys;
-    float4* tex_vals;
-    uint32_t tex_sentinel;         // key of an unused record, above every texel index
-    uint32_t* vtx_keys;
-    float4* vtx_vals;              // 2 per record: colour gradient, (u, v, 0, 0) gradient
-    uint32_t vtx_sentinel;
+    float4* tex_recs;              // 2 per pixel: dL/dsample, then cell position, flags and texture width
+    uint32_t tex_sentinel;         // key of a pixel without a texel, above every texel index
+    // ... and per block of pixels a run per triangle it shows
+    uint32_t total_blocks;
+    uint32_t* block_runs;          // [total_blocks]
+    uint32_t* run_mesh;            // [total_blocks][256] meshlet, ascending
+    uint8_t* run_tri;              // [total_blocks][256] triangle
+    uint8_t* run_same;             // [total_blocks][256] the block's other runs of the meshlet
+    float* run_sums;               // [total_blocks][256][18]
+    // the vertex gradients' work list
+    uint32_t* cells;               // [views][meshlets][8] a bit per cell of the view the meshlet shows in
+    uint32_t* cell_counts;         // [meshlets]
+    uint32_t* parts_done;          // [meshlets]
+    uint32_t* part_state;          // marked cells; parts
+    uint4* parts;                  // meshlet, part of it, its parts, its first part's place
+    float* part_sums;              // [parts][6][64]
+    uint32_t max_parts, part_cells, cell_blocks;
 };
 
 // Device buffers of one backward pass (owned by the context).
 struct DiffWorkspace {
-    size_t pixels = 0, texels = 0;
+    size_t pixels = 0, blocks = 0, meshlets = 0, marks_cap = 0;
     uint32_t* tex_keys = nullptr;
-    float4* tex_vals = nullptr;
-    uint32_t* vtx_keys = nullptr;
-    float4* vtx_vals = nullptr;
+    float4* tex_recs = nullptr;
+    float4* cells = nullptr;       // per run of equal texels, at its first record: three corners, flags and width
     uint32_t* sorted_keys = nullptr;
     uint32_t* sorted_idx = nullptr;
-    float4* part_first = nullptr;  // per 256-record tile, up to 2 float4 each
-    float4* part_last = nullptr;
-    uint32_t* key_last = nullptr;
+    uint8_t* parts = nullptr;      // per 256-record tile the pieces of runs that cross it
+    uint2* last = nullptr;         // per tile its last run (texel, first record) when that goes on
     uint32_t* spans = nullptr;
+    uint32_t* marks = nullptr;     // cells, parts_done, part_state
+    uint32_t* cell_counts = nullptr;
+    uint4* part_list = nullptr;
+    float* part_sums = nullptr;
+    uint32_t* block_runs = nullptr;
+    uint32_t* run_mesh = nullptr;
+    uint8_t* run_tri = nullptr;
+    uint8_t* run_same = nullptr;
+    float* run_sums = nullptr;
     void* sort_temp = nullptr;
     size_t sort_temp_bytes = 0;
 };
 
-hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels);
+hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks, size_t meshlets, size_t views);
 void diff_workspace_release(DiffWorkspace& w);
 hipError_t launch_diff_forward(const DiffParams& p, hipStream_t s, Profiler* prof);
 // grad_texels [num_texels], grad_uv [vertices], grad_color [vertices] are
 // overwritten (zeros where nothing contributes).
-hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_texels, uint32_t num_vertices,
-                                float4* grad_texels, float2* grad_uv, float4* grad_color, hipStream_t s,
-                                Profiler* prof);
+hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_texels, float4* grad_texels,
+                                float2* grad_uv, float4* grad_color, hipStream_t s, Profiler* prof);
 
 }  // namespace glimp

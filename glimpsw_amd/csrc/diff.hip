@@ -14,14 +14,27 @@
 // weights are continuous (texel centres at +0.5, clamped at the edges) so
 // that the output is differentiable in U and V.
 //
-// Backward: one pass over the pixels writes, per pixel, four texel records
-// (texel index, weight * dL/dsample) and three vertex records (vertex index,
-// barycentric weight * (dL/dcol, dL/dU, dL/dV)) into fixed slots. The
-// records are sorted by index with a stable radix sort, and every run of
-// equal indices is summed in slot order: in 256-record tiles by one thread
-// per run piece, then across tiles in tile order. The order of every
-// floating-point addition depends only on the inputs, so the gradients are
-// bitwise reproducible; no floating-point atomics are used.
+// Backward: one pass over the pixels (k_diff_pixels) splits the gradient in
+// two.
+//
+// Vertices. A block covers 16x16 pixels of one view; each of its waves sums,
+// per triangle it shows (a run), the 18 products of barycentric weight and
+// (dL/dcol, dL/dU, dL/dV) over the run's pixels in lane order, and marks in
+// which cells of a 16x16 grid over the view each of its meshlets shows.
+// k_diff_vertices walks a meshlet's marked cells in order, adds the meshlet's
+// runs per triangle and then the triangles' corners per vertex; a meshlet of
+// many cells is split into parts, added in order by the last one to finish.
+//
+// Texels. Each pixel leaves one record: its base texel (the cell's corner, or
+// the nearest texel), dL/dsample and the cell position. The pixels are sorted
+// by base texel with a stable radix sort; every run of equal texels is summed
+// in pixel order into the four corners of its cell, in 256-record tiles by
+// one thread per run piece, then across tiles in tile order. No two cells
+// share a corner of the same kind, so four passes add the corners to the
+// gradients, one kind at a time, without conflicts.
+//
+// The order of every floating-point addition depends only on the inputs, so
+// the gradients are bitwise reproducible; no floating-point atomics are used.
 #include <hip/hip_runtime.h>
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/iterator/counting_iterator.hpp>
@@ -36,7 +49,7 @@ constexpr uint32_t kTile = 256;
 
 struct PixelState {
     bool active;
-    uint32_t mi, vi[3];
+    uint32_t mi, tri, vi[3];
     float b1, b2, U, V;
     int32_t tex, level;
     bool linear;
@@ -82,6 +95,28 @@ __device__ __forceinline__ PixelSlot pixel_slot(const DiffParams& p, uint32_t t)
     return s;
 }
 
+// Pixel of thread `tid` of 16x16-pixel block b: 16 lanes are one 4x4 tile, a
+// wave 8x8 pixels (a compact area shows the fewest triangles).
+__device__ __forceinline__ PixelSlot block_slot(const DiffParams& p, uint32_t b, uint32_t tid, uint32_t& bx,
+                                                uint32_t& by) {
+    uint32_t lo = 0, hi = p.num_views;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (view_at(p, mid).block_base <= b) lo = mid; else hi = mid;
+    }
+    const DiffView& V = view_at(p, lo);
+    by = (b - V.block_base) / V.blocks_x;
+    bx = (b - V.block_base) - by * V.blocks_x;
+    const uint32_t tile = tid >> 4, q = tid & 15u;
+    PixelSlot s;
+    s.view = lo;
+    s.x = bx * 16 + ((tile >> 2) & 1u) * 8 + (tile & 1u) * 4 + (q & 3u);
+    s.y = by * 16 + (tile >> 3) * 8 + ((tile >> 1) & 1u) * 4 + (q >> 2);
+    s.inside = s.x < (uint32_t)V.width && s.y < (uint32_t)V.height;
+    s.tiled = s.inside ? ((s.x & ~3u) << 2) + (s.y & ~3u) * (uint32_t)V.width + q : 0u;
+    return s;
+}
+
 // Surface, barycentrics and sampler choices of pixel slot t (tiled order:
 // 16 lanes = one 4x4 tile of one view). Every lane of the wave must call it.
 __device__ void diff_pixel(const DiffParams& p, const PixelSlot& ps, PixelState& S) {
@@ -104,6 +139,7 @@ __device__ void diff_pixel(const DiffParams& p, const PixelSlot& ps, PixelState&
     if (active) {
         uint32_t tri;
         decode_surface(key, VW.draws, VW.num_draws, S.mi, tri);
+        S.tri = tri;
         const uint8_t* I = p.m.indices + (size_t)S.mi * 384;
         const float* P = p.m.positions + (size_t)S.mi * 192;
         float c[3][4], uv[3][2];
@@ -198,7 +234,7 @@ __device__ void diff_pixel(const DiffParams& p, const PixelSlot& ps, PixelState&
 struct SampleEval {
     float4 val, du, dv;
     uint64_t texel[4];
-    float w[4];
+    float fx, fy;
     int n;
 };
 
@@ -228,7 +264,6 @@ __device__ void sample_eval(const DiffParams& p, const PixelState& S, SampleEval
         const uint64_t Wm = D.width >> S.level;
         E.n = 1;
         E.texel[0] = base + (uint64_t)S.ty * Wm + (uint64_t)S.tx;
-        E.w[0] = 1.0f;
         E.val = p.texels[E.texel[0]];
         return;
     }
@@ -241,11 +276,9 @@ __device__ void sample_eval(const DiffParams& p, const PixelState& S, SampleEval
     E.texel[1] = base + y0 * D.width + x1;
     E.texel[2] = base + y1 * D.width + x0;
     E.texel[3] = base + y1 * D.width + x1;
+    E.fx = fx;
+    E.fy = fy;
     const float gx = 1.0f - fx, gy = 1.0f - fy;
-    E.w[0] = gx * gy;
-    E.w[1] = fx * gy;
-    E.w[2] = gx * fy;
-    E.w[3] = fx * fy;
     const float4 t00 = p.texels[E.texel[0]], t10 = p.texels[E.texel[1]];
     const float4 t01 = p.texels[E.texel[2]], t11 = p.texels[E.texel[3]];
     const float4 d0 = t10 - t00, d1 = t11 - t01;
@@ -282,129 +315,532 @@ __global__ void __launch_bounds__(256) k_diff_forward(DiffParams p) {
     p.out[out_index(p, ps)] = o;
 }
 
-// Per-pixel gradient records (fixed slots 4t.. and 3t..).
-__global__ void __launch_bounds__(256) k_diff_records(DiffParams p) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const PixelSlot ps = pixel_slot(p, t);
+// ---------------------------------------------------------------- backward: pixels
+
+constexpr uint32_t kBlockRuns = 256;   // most runs of a block of pixels: 64 a wave
+constexpr uint32_t kRunSums = 18;      // 3 corners x (colour, U, V)
+constexpr uint32_t kSplitParts = 32768;                    // most parts beyond one per meshlet
+constexpr uint32_t kPartGrid = 2048;   // 8 blocks a CU
+
+// Texel record flags
+constexpr uint32_t kTexLinear = 1u, kTexRight = 2u, kTexBelow = 4u;
+
+// Bound by the surface evaluation, as k_diff_forward, and 36 bytes a pixel of
+// texel records: 130 us for 2.76 M pixels of three 1280x720 views (forward
+// 67). Four texel and three vertex records a pixel, 188 bytes, took 233 us.
+// Run sums are per wave, not per block: a block-wide set of triangles cost
+// four barriers and a hash table (193 us). Growing a rectangle per meshlet
+// with atomic minima instead of marking cells took 177 us: the large
+// meshlets' corners are contended.
+__global__ void __launch_bounds__(256) k_diff_pixels(DiffParams p) {
+    __shared__ float s_val[8][256];              // b1, b2, gcol, gU, gV per pixel
+    __shared__ unsigned long long s_mask[kBlockRuns];      // a run's pixels in its wave
+    __shared__ uint32_t s_mesh[kBlockRuns], s_pos[kBlockRuns], s_count[4];
+    __shared__ uint8_t s_tri[kBlockRuns];
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), wid = tid >> 6;
+    uint32_t bx, by;
+    const PixelSlot ps = block_slot(p, blockIdx.x, tid, bx, by);
     PixelState S;
     diff_pixel(p, ps, S);
-    if (!ps.inside) return;
-    uint32_t tkeys[4] = { p.tex_sentinel, p.tex_sentinel, p.tex_sentinel, p.tex_sentinel };
-    float4 tvals[4] = { f4(0.0f), f4(0.0f), f4(0.0f), f4(0.0f) };
-    uint32_t vkeys[3] = { p.vtx_sentinel, p.vtx_sentinel, p.vtx_sentinel };
-    float4 vcol[3] = { f4(0.0f), f4(0.0f), f4(0.0f) }, vuv[3] = { f4(0.0f), f4(0.0f), f4(0.0f) };
-    if (S.active) {
-        SampleEval E;
-        sample_eval(p, S, E);
-        const float4 g = p.grad_out[out_index(p, ps)];
-        const float4 col = vertex_color(p, S);
-        const float4 gval = g * col;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (k < E.n) {
-                tkeys[k] = (uint32_t)E.texel[k];
-                tvals[k] = E.w[k] * gval;
+    if (ps.inside) {
+        const DiffView& V = view_at(p, ps.view);
+        const size_t t = (size_t)V.pixel_base + ps.tiled;
+        uint32_t texel = p.tex_sentinel;
+        if (S.active) {
+            SampleEval E;
+            sample_eval(p, S, E);
+            const float4 g = p.grad_out[out_index(p, ps)];
+            const float4 gval = g * vertex_color(p, S);
+            const float4 gcol = g * E.val;
+            if (E.n) {
+                texel = (uint32_t)E.texel[0];
+                uint32_t code = 0, width = 0;
+                float fx = 0.0f, fy = 0.0f;
+                if (E.n == 4) {
+                    code = kTexLinear | (S.ex ? kTexRight : 0u) | (S.ey ? kTexBelow : 0u);
+                    width = p.textures[S.tex].width;
+                    fx = E.fx;
+                    fy = E.fy;
+                }
+                p.tex_recs[2 * t] = gval;
+                p.tex_recs[2 * t + 1] = make_float4(fx, fy, __uint_as_float(code), __uint_as_float(width));
             }
+            s_val[0][tid] = S.b1;
+            s_val[1][tid] = S.b2;
+            s_val[2][tid] = gcol.x;
+            s_val[3][tid] = gcol.y;
+            s_val[4][tid] = gcol.z;
+            s_val[5][tid] = gcol.w;
+            s_val[6][tid] = dot4(gval, E.du);
+            s_val[7][tid] = dot4(gval, E.dv);
         }
-        const float gU = dot4(gval, E.du), gV = dot4(gval, E.dv);
-        const float4 gcol = g * E.val;
-        const float w[3] = { (1.0f - S.b1) - S.b2, S.b1, S.b2 };
+        p.tex_keys[t] = texel;
+    }
+    // the wave's pixels of each triangle: the first of them holds the mask
+    const bool active = S.active;          // only inside the view
+    unsigned long long todo = __ballot(active), mine = 0;
+    while (todo) {
+        const int l = __builtin_ctzll(todo);
+        const uint32_t m0 = (uint32_t)__builtin_amdgcn_readlane((int)S.mi, l);
+        const uint32_t t0 = (uint32_t)__builtin_amdgcn_readlane((int)S.tri, l);
+        const unsigned long long m = __ballot(active && S.mi == m0 && S.tri == t0);
+        if (lane == (uint32_t)l) mine = m;
+        todo &= ~m;
+    }
+    // the wave's runs in the order of their first pixels, the waves' one after another
+    const unsigned long long leaders = __ballot(mine != 0);
+    const uint32_t own = (uint32_t)__popcll(leaders);
+    if (lane == 0) s_count[wid] = own;
+    __syncthreads();
+    uint32_t first = 0, runs = 0;
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-            vkeys[k] = S.mi * 64 + S.vi[k];
-            vcol[k] = w[k] * gcol;
-            vuv[k] = make_float4(w[k] * gU, w[k] * gV, 0.0f, 0.0f);
+    for (uint32_t w = 0; w < 4; w++) {
+        if (w < wid) first += s_count[w];
+        runs += s_count[w];
+    }
+    if (mine) {
+        const uint32_t r = first + (uint32_t)__popcll(leaders & ((1ull << lane) - 1ull));
+        s_mask[r] = mine;
+        s_mesh[r] = S.mi;
+        s_tri[r] = (uint8_t)S.tri;
+    }
+    __syncthreads();
+    const size_t base = (size_t)blockIdx.x * kBlockRuns;
+    if (tid == 0) p.block_runs[blockIdx.x] = runs;
+    if (tid < runs) {
+        // runs are kept by meshlet, in that order within it
+        const uint32_t mesh = s_mesh[tid];
+        uint32_t pos = 0, same = 0;
+        for (uint32_t r = 0; r < runs; r++) {
+            const uint32_t o = s_mesh[r];
+            pos += (o < mesh || (o == mesh && r < tid)) ? 1u : 0u;
+            same += o == mesh ? 1u : 0u;
         }
+        s_pos[tid] = pos;
+        p.run_same[base + pos] = (uint8_t)(same - 1);
+        p.run_mesh[base + pos] = mesh;
+        p.run_tri[base + pos] = s_tri[tid];
+        // mark the meshlet's cell (a plain read first: nearly every block finds it marked)
+        const DiffView& V = view_at(p, ps.view);
+        const uint32_t cell = (by / V.cell_h) * 16 + bx / V.cell_w;
+        uint32_t* word = p.cells + ((size_t)ps.view * p.m.count + mesh) * 8 + (cell >> 5);
+        const uint32_t bit = 1u << (cell & 31u);
+        if (!(__atomic_load_n(word, __ATOMIC_RELAXED) & bit)) atomicOr(word, bit);
     }
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        p.tex_keys[(size_t)t * 4 + k] = tkeys[k];
-        p.tex_vals[(size_t)t * 4 + k] = tvals[k];
-    }
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        p.vtx_keys[(size_t)t * 3 + k] = vkeys[k];
-        p.vtx_vals[((size_t)t * 3 + k) * 2 + 0] = vcol[k];
-        p.vtx_vals[((size_t)t * 3 + k) * 2 + 1] = vuv[k];
+    __syncthreads();
+    // the wave's (run, value) pairs over its lanes: three corner sums each,
+    // over the run's pixels in order
+    for (uint32_t i = lane; i < own * 6; i += 64) {
+        const uint32_t q = i / 6, c = i - q * 6, r = first + q;
+        const float *val = &s_val[2 + c][wid * 64], *w1 = &s_val[0][wid * 64], *w2 = &s_val[1][wid * 64];
+        float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
+        auto add = [&](float v, float b1, float b2) {
+            a0 = __builtin_fmaf((1.0f - b1) - b2, v, a0);
+            a1 = __builtin_fmaf(b1, v, a1);
+            a2 = __builtin_fmaf(b2, v, a2);
+        };
+        unsigned long long m = s_mask[r];
+        while (m) {       // two pixels a step: their reads overlap
+            const uint32_t j = (uint32_t)__builtin_ctzll(m);
+            m &= m - 1ull;
+            const bool two = m != 0;
+            const uint32_t k = two ? (uint32_t)__builtin_ctzll(m) : j;
+            m &= m - 1ull;     // 0 stays 0
+            const float vj = val[j], b1j = w1[j], b2j = w2[j], vk = val[k], b1k = w1[k], b2k = w2[k];
+            add(vj, b1j, b2j);
+            if (two) add(vk, b1k, b2k);
+        }
+        float* out = p.run_sums + (base + s_pos[r]) * kRunSums + c;
+        out[0] = a0;
+        out[6] = a1;
+        out[12] = a2;
     }
 }
 
-// Gradient outputs of a segmented reduction: K float4 per record.
-struct TexelOut {
-    float4* grad;
-    __device__ void write(uint32_t key, const float4* v) const { grad[key] = v[0]; }
-};
-struct VertexOut {
-    float4* color;
-    float2* uv;
-    __device__ void write(uint32_t key, const float4* v) const {
-        color[key] = v[0];
-        uv[key] = make_float2(v[1].x, v[1].y);
+// ---------------------------------------------------------------- backward: vertices
+
+// Marked cells of each meshlet, and of all together (they set the part size).
+__global__ void __launch_bounds__(256) k_count_cells(DiffParams p) {
+    __shared__ uint32_t s_total;
+    const uint32_t mi = blockIdx.x * 256 + threadIdx.x;
+    if (threadIdx.x == 0) s_total = 0;
+    __syncthreads();
+    uint32_t n = 0;
+    if (mi < p.m.count) {
+        for (uint32_t v = 0; v < p.num_views; v++) {
+            const uint4* w = reinterpret_cast<const uint4*>(p.cells + ((size_t)v * p.m.count + mi) * 8);
+            const uint4 a = w[0], b = w[1];
+            n += __popc(a.x) + __popc(a.y) + __popc(a.z) + __popc(a.w) + __popc(b.x) + __popc(b.y) + __popc(b.z) +
+                 __popc(b.w);
+        }
+        p.cell_counts[mi] = n;
+    }
+    if (n) atomicAdd(&s_total, n);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_total) atomicAdd(&p.part_state[0], s_total);
+}
+
+// Cells of a part: about kPartBlocks pixel blocks, more when that would
+// make more than max_parts parts.
+__device__ __forceinline__ uint32_t part_cells(const DiffParams& p) {
+    const uint32_t room = p.max_parts - p.m.count;      // every meshlet's last part may be a short one
+    return max(p.part_cells, (p.part_state[0] + room - 1) / room);
+}
+
+// The parts of every meshlet (one for a meshlet that shows nowhere: it writes
+// zeros); the order of the list does not matter.
+__global__ void __launch_bounds__(256) k_list_parts(DiffParams p) {
+    const uint32_t mi = blockIdx.x * 256 + threadIdx.x;
+    if (mi >= p.m.count) return;
+    const uint32_t g = part_cells(p);
+    const uint32_t n = max(1u, (p.cell_counts[mi] + g - 1) / g);
+    const uint32_t at = atomicAdd(&p.part_state[1], n);
+    for (uint32_t k = 0; k < n; k++) p.parts[at + k] = make_uint4(mi, k, n, at);
+}
+
+// One part a block at a time: the runs of its cells' pixel blocks, 256 blocks
+// at a time, are listed in block order and taken in rounds of kRoundRuns:
+// their sums are staged in LDS, each triangle's are a bit mask, and a thread
+// per (triangle, sum) adds them in order. 2.76 M pixels, 6,000 meshlets: 137 us
+// (sorting and reducing 8.3 M vertex records took 574), most of it the
+// meshlets at the eye, whose parts list thousands of runs; one block per
+// meshlet took 360 us with a linear search for the runs and a thread per
+// triangle comparing every run's.
+constexpr uint32_t kRoundRuns = 128;
+constexpr uint32_t kPartBlocks = 256;
+
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* s_wave, uint32_t& total) {
+    const uint32_t lane = __lane_id(), wid = threadIdx.x >> 6;
+    uint32_t incl = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)incl, d);
+        if (lane >= (uint32_t)d) incl += o;
+    }
+    if (lane == 63) s_wave[wid] = incl;
+    __syncthreads();
+    uint32_t first = incl - v;
+    total = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 4; q++) {
+        if (q < wid) first += s_wave[q];
+        total += s_wave[q];
+    }
+    __syncthreads();
+    return first;
+}
+
+__global__ void __launch_bounds__(256) k_diff_vertices(DiffParams p, float4* grad_color, float2* grad_uv) {
+    __shared__ float s_sum[128][kRunSums];             // per triangle
+    __shared__ float s_stage[kRoundRuns][kRunSums];
+    __shared__ size_t s_list[kRoundRuns];
+    __shared__ unsigned long long s_bits[128][2];      // a triangle's runs of the round
+    __shared__ unsigned long long s_corner[64][3][2];  // the triangles a vertex is corner k of
+    __shared__ uint32_t s_seen[128], s_ntris, s_wave[4], s_last;
+    __shared__ uint8_t s_tris[128];
+    __shared__ uint32_t s_cells[kPartBlocks];          // view << 8 | cell
+    const uint32_t tid = threadIdx.x, lane = __lane_id(), wid = tid >> 6;
+    if (tid < 128) {
+        s_bits[tid][0] = s_bits[tid][1] = 0ull;
+        s_seen[tid] = 0;
+    }
+    if (tid == 0) s_ntris = 0;
+    const uint32_t nparts = p.part_state[1], group = part_cells(p);
+    for (uint32_t item = blockIdx.x; item < nparts; item += gridDim.x) {
+        const uint4 part = p.parts[item];
+        const uint32_t mi = part.x, cells = p.cell_counts[mi];
+        const uint32_t c_lo = part.y * group, c_hi = min(cells, c_lo + group);
+        if (c_lo < c_hi) {
+            for (uint32_t i = tid; i < 128 * kRunSums; i += 256) s_sum[i / kRunSums][i % kRunSums] = 0.0f;
+            for (uint32_t i = tid; i < 384; i += 256) s_corner[i / 6][(i / 2) % 3][i & 1] = 0ull;
+            __syncthreads();
+            const uint32_t nt = min((uint32_t)p.m.num_triangles[mi], 128u);
+            for (uint32_t i = tid; i < 384; i += 256) {
+                const uint32_t k = i >> 7, q = i & 127u, v = p.m.indices[(size_t)mi * 384 + i];
+                if (q < nt && v < 64) atomicOr(&s_corner[v][k][q >> 6], 1ull << (q & 63u));
+            }
+        }
+        for (uint32_t g0 = c_lo; g0 < c_hi; g0 += kPartBlocks) {
+            const uint32_t g1 = min(c_hi, g0 + kPartBlocks);
+            // cells [g0, g1) of the meshlet's, in (view, cell) order
+            uint32_t seen = 0;
+            for (uint32_t v0 = 0; v0 < p.num_views && seen < g1; v0 += 32) {
+                const uint32_t v = v0 + (tid >> 3);
+                uint32_t w = v < p.num_views ? p.cells[((size_t)v * p.m.count + mi) * 8 + (tid & 7u)] : 0u;
+                uint32_t total = 0;
+                uint32_t rank = seen + block_scan((uint32_t)__popc(w), s_wave, total);
+                for (; w && rank < g1; w &= w - 1, rank++)
+                    if (rank >= g0) s_cells[rank - g0] = (v << 8) | (tid & 7u) * 32 + (uint32_t)__builtin_ctz(w);
+                seen += total;
+            }
+            __syncthreads();
+            const uint32_t candidates = (g1 - g0) * p.cell_blocks;
+            for (uint32_t c0 = 0; c0 < candidates; c0 += 256) {
+                const uint32_t c = c0 + tid;
+                size_t base = 0;
+                uint32_t found = 0;
+                if (c < candidates) {
+                    const uint32_t i = c / p.cell_blocks, q = c - i * p.cell_blocks;
+                    const uint32_t vc = s_cells[i];
+                    const DiffView& V = view_at(p, vc >> 8);
+                    const uint32_t dy = q / V.cell_w, dx = q - dy * V.cell_w;
+                    const uint32_t x = (vc & 15u) * V.cell_w + dx, y = ((vc >> 4) & 15u) * V.cell_h + dy;
+                    if (dy < V.cell_h && x < V.blocks_x && y < V.blocks_y) {
+                        const uint32_t b = V.block_base + y * V.blocks_x + x;
+                        base = (size_t)b * kBlockRuns;
+                        const uint32_t runs = p.block_runs[b];
+                        // the runs are sorted by meshlet: find its first
+                        uint32_t at = 0;
+                        for (uint32_t len = runs; len > 0;) {
+                            const uint32_t half_len = len >> 1;
+                            const bool up = p.run_mesh[base + at + half_len] < mi;
+                            at = up ? at + half_len + 1 : at;
+                            len = up ? len - half_len - 1 : half_len;
+                        }
+                        if (at < runs && p.run_mesh[base + at] == mi) found = p.run_same[base + at] + 1u;
+                        base += at;
+                    }
+                }
+                uint32_t total = 0;
+                const uint32_t first = block_scan(found, s_wave, total);
+                for (uint32_t r0 = 0; r0 < total; r0 += kRoundRuns) {
+                    const uint32_t lo = max(first, r0), hi = min(first + found, r0 + kRoundRuns);
+                    for (uint32_t k = lo; k < hi; k++) s_list[k - r0] = base + (k - first);
+                    __syncthreads();
+                    const uint32_t n = min(kRoundRuns, total - r0);
+                    if (tid < n) {
+                        // the round's runs of each triangle, and the triangles that have some
+                        const uint32_t k = p.run_tri[s_list[tid]] & 127u;
+                        atomicOr(&s_bits[k][tid >> 6], 1ull << (tid & 63u));
+                        if (atomicOr(&s_seen[k], 1u) == 0) s_tris[atomicAdd(&s_ntris, 1u)] = (uint8_t)k;
+                    }
+                    for (uint32_t i = tid; i < n * kRunSums; i += 256) {
+                        const uint32_t e = i / kRunSums, q = i - e * kRunSums;
+                        s_stage[e][q] = p.run_sums[s_list[e] * kRunSums + q];
+                    }
+                    __syncthreads();
+                    const uint32_t ntris = s_ntris;
+                    for (uint32_t i = tid; i < ntris * kRunSums; i += 256) {
+                        const uint32_t e = i / kRunSums, q = i - e * kRunSums, k = s_tris[e];
+                        float a = s_sum[k][q];
+#pragma unroll
+                        for (uint32_t w = 0; w < 2; w++) {
+                            unsigned long long m = s_bits[k][w];
+                            while (m) {        // two runs a step: their reads overlap
+                                const uint32_t j0 = w * 64 + (uint32_t)__builtin_ctzll(m);
+                                m &= m - 1ull;
+                                const bool two = m != 0;
+                                const uint32_t j1 = two ? w * 64 + (uint32_t)__builtin_ctzll(m) : j0;
+                                m &= m - 1ull;     // 0 stays 0
+                                const float v0 = s_stage[j0][q], v1 = s_stage[j1][q];
+                                a += v0;
+                                if (two) a += v1;
+                            }
+                        }
+                        s_sum[k][q] = a;
+                    }
+                    __syncthreads();
+                    if (tid < ntris) {
+                        const uint32_t k = s_tris[tid];
+                        s_bits[k][0] = s_bits[k][1] = 0ull;
+                        s_seen[k] = 0;
+                    }
+                    if (tid == 0) s_ntris = 0;
+                    __syncthreads();
+                }
+            }
+        }
+        // triangles' corners to vertices: lane = vertex; wave 0-3: channels
+        // 0-1, 2-3, 4 and 5 of (colour, U, V)
+        const uint32_t ch = wid < 2 ? wid * 2 : wid + 2;
+        float g0 = 0.0f, g1 = 0.0f;
+        if (c_lo < c_hi) {
+#pragma unroll
+            for (uint32_t k = 0; k < 3; k++) {
+#pragma unroll
+                for (uint32_t w = 0; w < 2; w++) {
+                    for (unsigned long long m = s_corner[lane][k][w]; m; m &= m - 1ull) {
+                        const uint32_t q = w * 64 + (uint32_t)__builtin_ctzll(m);
+                        g0 += s_sum[q][k * 6 + ch];
+                        if (wid < 2) g1 += s_sum[q][k * 6 + ch + 1];
+                    }
+                }
+            }
+        }
+        bool write = true;
+        if (part.z > 1) {
+            // a part of several: the last to finish adds them in order
+            float* mine = p.part_sums + (size_t)item * 384;
+            mine[ch * 64 + lane] = g0;
+            if (wid < 2) mine[(ch + 1) * 64 + lane] = g1;
+            __threadfence();
+            __syncthreads();
+            if (tid == 0) s_last = atomicAdd(&p.parts_done[mi], 1u);
+            __syncthreads();
+            write = s_last == part.z - 1;
+            if (write) {
+                __threadfence();
+                g0 = g1 = 0.0f;
+                for (uint32_t k = 0; k < part.z; k++) {
+                    const float* o = p.part_sums + (size_t)(part.w + k) * 384;
+                    g0 += __hip_atomic_load(o + ch * 64 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (wid < 2) g1 += __hip_atomic_load(o + (ch + 1) * 64 + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+        }
+        if (write) {
+            const size_t vtx = (size_t)mi * 64 + lane;
+            if (wid < 2) reinterpret_cast<float2*>(grad_color + vtx)[wid] = make_float2(g0, g1);
+            else reinterpret_cast<float*>(grad_uv + vtx)[wid - 2] = g0;
+        }
+        __syncthreads();       // s_sum, s_idx, s_last
+    }
+}
+
+// ---------------------------------------------------------------- backward: texels
+
+// Gradients of the four corners of a cell, and the cell's flags and texture
+// width (flags 0: a nearest texel only).
+struct CellSum {
+    float4 c[4];
+    uint32_t code, width;
+
+    __device__ void clear() {
+#pragma unroll
+        for (int k = 0; k < 4; k++) c[k] = f4(0.0f);
+        code = width = 0;
+    }
+    // a pixel's record: dL/dsample g, cell position, flags, texture width
+    __device__ void add(float4 g, float fx, float fy, uint32_t cd, uint32_t w) {
+        if (!(cd & kTexLinear)) {
+            c[0] = add4(c[0], g);
+            return;
+        }
+        const float gx = 1.0f - fx, gy = 1.0f - fy;
+        c[0] = fma4(gx * gy, g, c[0]);
+        c[1] = fma4(fx * gy, g, c[1]);
+        c[2] = fma4(gx * fy, g, c[2]);
+        c[3] = fma4(fx * fy, g, c[3]);
+        code = cd;
+        width = w;
+    }
+    __device__ void add(const CellSum& o) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) c[k] = add4(c[k], o.c[k]);
+        if (o.code) {
+            code = o.code;
+            width = o.width;
+        }
+    }
+    // corners past the texture's edge are the cell's own (their weight is 0)
+    __device__ void fold() {
+        if (!code) return;
+        if (!(code & kTexRight)) {
+            c[0] = add4(c[0], c[1]);
+            c[2] = add4(c[2], c[3]);
+        }
+        if (!(code & kTexBelow)) {
+            c[0] = add4(c[0], c[2]);
+            c[1] = add4(c[1], c[3]);
+        }
+    }
+    // the base texel's gradient; the other corners for k_tex_corner
+    __device__ void write(uint32_t key, float4* grad, float4* cells, size_t start) {
+        fold();
+        grad[key] = c[0];
+        float4* o = cells + start * 4;
+        if (code) {
+            o[0] = c[1];
+            o[1] = c[2];
+            o[2] = c[3];
+        }
+        o[3] = make_float4(__uint_as_float(code), __uint_as_float(width), 0.0f, 0.0f);
     }
 };
 
-template <int K, class Out>
-__global__ void __launch_bounds__(kTile) k_seg_reduce(const uint32_t* keys, const uint32_t* idx, const float4* vals,
-                                                      uint32_t n, uint32_t sentinel, Out out, float4* part_first,
-                                                      float4* part_last, uint32_t* key_last, uint32_t* spans) {
+// One thread per run piece of a tile of kTile sorted records: 111 us for 2.76 M
+// records, bound by the gather of 32 bytes a record in texel order. With the
+// sort (140 us, 2.76 M keys instead of 11 M) and the corners (47 us) the
+// texel gradients take 298 us, 504 before.
+__global__ void __launch_bounds__(kTile) k_tex_reduce(const uint32_t* keys, const uint32_t* idx, const float4* recs,
+                                                      uint32_t n, uint32_t sentinel, float4* grad, float4* cells,
+                                                      CellSum* part_first, CellSum* part_last, uint2* last,
+                                                      uint32_t* spans) {
     __shared__ uint32_t skey[kTile];
-    __shared__ float4 sval[kTile][K];
+    __shared__ float4 sval[kTile], spos[kTile];
     const uint32_t tile = blockIdx.x, tid = threadIdx.x;
     const uint32_t i0 = tile * kTile;
     const uint32_t cnt = min(kTile, n - i0);
     if (tid < cnt) {
-        skey[tid] = keys[i0 + tid];
-        const uint32_t r = idx[i0 + tid];
-#pragma unroll
-        for (int k = 0; k < K; k++) sval[tid][k] = vals[(size_t)r * K + k];
+        const uint32_t key = keys[i0 + tid];
+        skey[tid] = key;
+        if (key != sentinel) {
+            const size_t r = idx[i0 + tid];
+            sval[tid] = recs[2 * r];
+            spos[tid] = recs[2 * r + 1];
+        }
     }
     __syncthreads();
     if (tid >= cnt) return;
     const uint32_t key = skey[tid];
-    if (key == sentinel) return;
+    if (key == sentinel) {
+        if (tid == cnt - 1) last[tile] = make_uint2(sentinel, 0u);
+        return;
+    }
     const uint32_t prev = tid ? skey[tid - 1] : (i0 ? keys[i0 - 1] : sentinel);
     if (tid && prev == key) return;   // not the first record of a piece
-    float4 acc[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) acc[k] = sval[tid][k];
-    uint32_t j = tid + 1;
+    CellSum acc;
+    acc.clear();
+    uint32_t j = tid;
     for (; j < cnt && skey[j] == key; j++) {
-#pragma unroll
-        for (int k = 0; k < K; k++) acc[k] = add4(acc[k], sval[j][k]);
+        const float4 q = spos[j];
+        acc.add(sval[j], q.x, q.y, __float_as_uint(q.z), __float_as_uint(q.w));
     }
     const bool starts_here = !(tid == 0 && prev == key);
     const bool cont_next = j == cnt && i0 + cnt < n && keys[i0 + cnt] == key;
+    if (j == cnt) last[tile] = starts_here && cont_next ? make_uint2(key, i0 + tid) : make_uint2(sentinel, 0u);
     if (starts_here && !cont_next) {
-        out.write(key, acc);
+        acc.write(key, grad, cells, i0 + tid);
     } else if (starts_here) {
-#pragma unroll
-        for (int k = 0; k < K; k++) part_last[(size_t)tile * K + k] = acc[k];
-        key_last[tile] = key;
+        part_last[tile] = acc;
     } else {
-#pragma unroll
-        for (int k = 0; k < K; k++) part_first[(size_t)tile * K + k] = acc[k];
+        part_first[tile] = acc;
         spans[tile] = cont_next ? 1u : 0u;
     }
 }
 
 // Runs that cross tiles: the tile where a run starts adds the pieces of the
 // following tiles in tile order.
-template <int K, class Out>
-__global__ void k_seg_fixup(uint32_t tiles, uint32_t sentinel, Out out, const float4* part_first,
-                            const float4* part_last, const uint32_t* key_last, const uint32_t* spans) {
+__global__ void k_tex_fixup(uint32_t tiles, uint32_t sentinel, float4* grad, float4* cells,
+                            const CellSum* part_first, const CellSum* part_last, const uint2* last,
+                            const uint32_t* spans) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= tiles) return;
-    const uint32_t key = key_last[t];
-    if (key == sentinel) return;
-    float4 acc[K];
-#pragma unroll
-    for (int k = 0; k < K; k++) acc[k] = part_last[(size_t)t * K + k];
+    const uint2 l = last[t];
+    if (l.x == sentinel) return;
+    CellSum acc = part_last[t];
     for (uint32_t u = t + 1; u < tiles; u++) {
-#pragma unroll
-        for (int k = 0; k < K; k++) acc[k] = add4(acc[k], part_first[(size_t)u * K + k]);
+        acc.add(part_first[u]);
         if (!spans[u]) break;
     }
-    out.write(key, acc);
+    acc.write(l.x, grad, cells, l.y);
+}
+
+// Adds the runs' corners of one kind (1 right, 2 below, 3 below right) to the
+// gradients: different cells have different corners of a kind.
+template <int Corner>
+__global__ void __launch_bounds__(256) k_tex_corner(const uint32_t* keys, uint32_t n, uint32_t sentinel,
+                                                    const float4* cells, float4* grad) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t key = keys[i];
+    if (key == sentinel || (i && keys[i - 1] == key)) return;
+    const float4 h = cells[(size_t)i * 4 + 3];
+    const uint32_t code = __float_as_uint(h.x), width = __float_as_uint(h.y);
+    constexpr uint32_t need = Corner == 1 ? kTexRight : (Corner == 2 ? kTexBelow : kTexRight | kTexBelow);
+    if ((code & need) != need) return;
+    const size_t at = (size_t)key + (Corner & 1 ? 1u : 0u) + (Corner & 2 ? width : 0u);
+    grad[at] = add4(grad[at], cells[(size_t)i * 4 + (Corner - 1)]);
 }
 
 __global__ void k_fill_u32(uint32_t* p, size_t n, uint32_t v) {
@@ -436,43 +872,51 @@ hipError_t fill_zero(void* p, size_t floats, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int K, class Out>
-hipError_t reduce_records(DiffWorkspace& w, const uint32_t* keys, const float4* vals, uint32_t n, uint32_t sentinel,
-                          Out out, hipStream_t s) {
-    size_t bytes = w.sort_temp_bytes;
-    hipError_t e = rocprim::radix_sort_pairs(w.sort_temp, bytes, keys, w.sorted_keys,
-                                             rocprim::counting_iterator<uint32_t>(0), w.sorted_idx, n, 0,
-                                             bits_for(sentinel), s);
-    if (e != hipSuccess) return e;
-    const uint32_t tiles = (n + kTile - 1) / kTile;
-    hipLaunchKernelGGL(k_fill_u32, dim3(std::min<uint32_t>((tiles + 255) / 256, 4096u)), dim3(256), 0, s, w.key_last,
-                       (size_t)tiles, sentinel);
-    hipLaunchKernelGGL((k_seg_reduce<K, Out>), dim3(tiles), dim3(kTile), 0, s, w.sorted_keys, w.sorted_idx, vals, n,
-                       sentinel, out, w.part_first, w.part_last, w.key_last, w.spans);
-    hipLaunchKernelGGL((k_seg_fixup<K, Out>), dim3((tiles + 255) / 256), dim3(256), 0, s, tiles, sentinel, out,
-                       w.part_first, w.part_last, w.key_last, w.spans);
-    return hipGetLastError();
-}
-
 }  // namespace
 
-hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels) {
+hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks, size_t meshlets, size_t views) {
+    hipError_t e = hipSuccess;
+    // cells, then the counters that start at zero with them
+    const size_t marks = views * meshlets * 8 + meshlets + 4;
+    if (marks > w.marks_cap) {
+        w.marks_cap = 0;
+        e = grow(w.marks, marks);
+        if (e != hipSuccess) return e;
+        w.marks_cap = marks;
+    }
+    if (meshlets > w.meshlets) {
+        w.meshlets = 0;
+        e = grow(w.cell_counts, meshlets);
+        if (e == hipSuccess) e = grow(w.part_list, meshlets + kSplitParts);
+        if (e == hipSuccess) e = grow(w.part_sums, (meshlets + kSplitParts) * 384);
+        if (e != hipSuccess) return e;
+        w.meshlets = meshlets;
+    }
+    if (blocks > w.blocks) {
+        w.blocks = 0;
+        e = grow(w.block_runs, blocks);
+        if (e == hipSuccess) e = grow(w.run_mesh, blocks * kBlockRuns);
+        if (e == hipSuccess) e = grow(w.run_tri, blocks * kBlockRuns);
+        if (e == hipSuccess) e = grow(w.run_same, blocks * kBlockRuns);
+        if (e == hipSuccess) e = grow(w.run_sums, blocks * kBlockRuns * kRunSums);
+        if (e != hipSuccess) return e;
+        w.blocks = blocks;
+    }
     if (pixels <= w.pixels) return hipSuccess;
-    const size_t nt = pixels * 4, nv = pixels * 3, tiles = (nt + kTile - 1) / kTile;
-    hipError_t e = grow(w.tex_keys, nt);
-    if (e == hipSuccess) e = grow(w.tex_vals, nt);
-    if (e == hipSuccess) e = grow(w.vtx_keys, nv);
-    if (e == hipSuccess) e = grow(w.vtx_vals, nv * 2);
-    if (e == hipSuccess) e = grow(w.sorted_keys, nt);
-    if (e == hipSuccess) e = grow(w.sorted_idx, nt);
-    if (e == hipSuccess) e = grow(w.part_first, tiles * 2);
-    if (e == hipSuccess) e = grow(w.part_last, tiles * 2);
-    if (e == hipSuccess) e = grow(w.key_last, tiles);
+    const size_t tiles = (pixels + kTile - 1) / kTile;
+    w.pixels = 0;
+    e = grow(w.tex_keys, pixels);
+    if (e == hipSuccess) e = grow(w.tex_recs, pixels * 2);
+    if (e == hipSuccess) e = grow(w.cells, pixels * 4);
+    if (e == hipSuccess) e = grow(w.sorted_keys, pixels);
+    if (e == hipSuccess) e = grow(w.sorted_idx, pixels);
+    if (e == hipSuccess) e = grow(w.parts, tiles * 2 * sizeof(CellSum));
+    if (e == hipSuccess) e = grow(w.last, tiles);
     if (e == hipSuccess) e = grow(w.spans, tiles);
     if (e != hipSuccess) return e;
     size_t bytes = 0;
     e = rocprim::radix_sort_pairs(nullptr, bytes, w.tex_keys, w.sorted_keys, rocprim::counting_iterator<uint32_t>(0),
-                                  w.sorted_idx, (uint32_t)nt, 0, 32, (hipStream_t)0);
+                                  w.sorted_idx, (uint32_t)pixels, 0, 32, (hipStream_t)0);
     if (e != hipSuccess) return e;
     if (w.sort_temp) (void)hipFree(w.sort_temp);
     w.sort_temp = nullptr;
@@ -484,8 +928,9 @@ hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels) {
 }
 
 void diff_workspace_release(DiffWorkspace& w) {
-    void* ptrs[] = { w.tex_keys, w.tex_vals, w.vtx_keys, w.vtx_vals, w.sorted_keys, w.sorted_idx,
-                     w.part_first, w.part_last, w.key_last, w.spans, w.sort_temp };
+    void* ptrs[] = { w.tex_keys, w.tex_recs, w.cells, w.sorted_keys, w.sorted_idx, w.parts,
+                     w.last,     w.spans,    w.marks, w.block_runs,  w.run_mesh,   w.run_tri, w.run_same, w.run_sums, w.sort_temp,
+                     w.cell_counts, w.part_list, w.part_sums };
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     w = DiffWorkspace();
@@ -497,37 +942,68 @@ hipError_t launch_diff_forward(const DiffParams& p, hipStream_t s, Profiler* pro
     return hipGetLastError();
 }
 
-hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_texels, uint32_t num_vertices,
-                                float4* grad_texels, float2* grad_uv, float4* grad_color, hipStream_t s,
-                                Profiler* prof) {
+hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_texels, float4* grad_texels,
+                                float2* grad_uv, float4* grad_color, hipStream_t s, Profiler* prof) {
     const uint32_t n = p.total_pixels;
     p.tex_keys = w.tex_keys;
-    p.tex_vals = w.tex_vals;
-    p.vtx_keys = w.vtx_keys;
-    p.vtx_vals = w.vtx_vals;
+    p.tex_recs = w.tex_recs;
     p.tex_sentinel = (uint32_t)num_texels;
-    p.vtx_sentinel = num_vertices;
+    const size_t cell_words = (size_t)p.num_views * p.m.count * 8;
+    p.cells = w.marks;
+    p.parts_done = w.marks + cell_words;
+    p.part_state = p.parts_done + p.m.count;
+    p.cell_counts = w.cell_counts;
+    p.parts = w.part_list;
+    p.part_sums = w.part_sums;
+    p.max_parts = p.m.count + kSplitParts;
+    p.part_cells = std::max(1u, kPartBlocks / p.cell_blocks);
+    p.block_runs = w.block_runs;
+    p.run_mesh = w.run_mesh;
+    p.run_tri = w.run_tri;
+    p.run_same = w.run_same;
+    p.run_sums = w.run_sums;
     hipError_t e;
     {
         Profiler::Scope sc(prof, "diff_zero_grads", s);
         e = fill_zero(grad_texels, num_texels * 4, s);
-        if (e == hipSuccess) e = fill_zero(grad_uv, (size_t)num_vertices * 2, s);
-        if (e == hipSuccess) e = fill_zero(grad_color, (size_t)num_vertices * 4, s);
+        if (e != hipSuccess) return e;
+        const size_t words = cell_words + p.m.count + 4;
+        hipLaunchKernelGGL(k_fill_u32, dim3((uint32_t)std::min<size_t>((words + 255) / 256, 4096)), dim3(256), 0, s,
+                           w.marks, words, 0u);
+        e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    launch_kernel(prof, "diff_records", k_diff_records, dim3((n + 255) / 256), dim3(256), 0, s, p);
+    launch_kernel(prof, "diff_pixels", k_diff_pixels, dim3(p.total_blocks), dim3(256), 0, s, p);
+    if (p.m.count) {
+        const uint32_t mb = (p.m.count + 255) / 256;
+        launch_kernel(prof, "diff_cells", k_count_cells, dim3(mb), dim3(256), 0, s, p);
+        launch_kernel(prof, "diff_parts", k_list_parts, dim3(mb), dim3(256), 0, s, p);
+        launch_kernel(prof, "diff_vertices", k_diff_vertices, dim3(kPartGrid), dim3(256), 0, s, p, grad_color, grad_uv);
+    }
     e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || !num_texels) return e;
     {
-        Profiler::Scope sc(prof, "diff_reduce_texels", s);
-        e = reduce_records<1>(w, w.tex_keys, w.tex_vals, n * 4, p.tex_sentinel, TexelOut{ grad_texels }, s);
+        Profiler::Scope sc(prof, "diff_sort_texels", s);
+        size_t bytes = w.sort_temp_bytes;
+        e = rocprim::radix_sort_pairs(w.sort_temp, bytes, w.tex_keys, w.sorted_keys,
+                                      rocprim::counting_iterator<uint32_t>(0), w.sorted_idx, n, 0,
+                                      bits_for(p.tex_sentinel), s);
         if (e != hipSuccess) return e;
     }
-    {
-        Profiler::Scope sc(prof, "diff_reduce_vertices", s);
-        e = reduce_records<2>(w, w.vtx_keys, w.vtx_vals, n * 3, p.vtx_sentinel, VertexOut{ grad_color, grad_uv }, s);
-    }
-    return e;
+    const uint32_t tiles = (n + kTile - 1) / kTile, blocks = (n + 255) / 256;
+    CellSum* part_first = reinterpret_cast<CellSum*>(w.parts);
+    CellSum* part_last = part_first + tiles;
+    launch_kernel(prof, "diff_texels", k_tex_reduce, dim3(tiles), dim3(kTile), 0, s, w.sorted_keys, w.sorted_idx,
+                  w.tex_recs, n, p.tex_sentinel, grad_texels, w.cells, part_first, part_last, w.last, w.spans);
+    launch_kernel(prof, "diff_texels_fixup", k_tex_fixup, dim3((tiles + 255) / 256), dim3(256), 0, s, tiles,
+                  p.tex_sentinel, grad_texels, w.cells, part_first, part_last, w.last, w.spans);
+    launch_kernel(prof, "diff_corner_1", k_tex_corner<1>, dim3(blocks), dim3(256), 0, s, w.sorted_keys, n,
+                  p.tex_sentinel, w.cells, grad_texels);
+    launch_kernel(prof, "diff_corner_2", k_tex_corner<2>, dim3(blocks), dim3(256), 0, s, w.sorted_keys, n,
+                  p.tex_sentinel, w.cells, grad_texels);
+    launch_kernel(prof, "diff_corner_3", k_tex_corner<3>, dim3(blocks), dim3(256), 0, s, w.sorted_keys, n,
+                  p.tex_sentinel, w.cells, grad_texels);
+    return hipGetLastError();
 }
 
 }  // namespace glimp
