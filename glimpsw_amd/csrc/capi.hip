@@ -338,6 +338,21 @@ int glimp_scene_create(glimp_context* c, const glimp_meshlets_desc* d, glimp_sce
     up((uint32_t**)&s->m.texcoords, d->texcoords, n * 64);
     up((uint32_t**)&s->m.normal_tangents, d->normal_tangents, n * 64);
     up((uint8_t**)&s->m.indices, d->indices, n * 384);
+    if (e == hipSuccess && n) {
+        // one allocation for the gather arrays, filled before the scene is
+        // handed out (any stream may use it then)
+        float4* g = nullptr;
+        e = dev_alloc(&g, n * (3 * 64 + 32));
+        if (e == hipSuccess) {
+            s->buffers.push_back(g);
+            s->m.vertices = g;
+            s->m.normals = g + n * 64;
+            s->m.tangents = g + n * 128;
+            s->m.triangles = reinterpret_cast<const uint32_t*>(g + n * 192);
+            e = launch_expand_meshlets(s->m, c->approx(), nullptr);
+        }
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    }
     if (e != hipSuccess) {
         glimp_scene_destroy(s);
         return fail(GLIMP_E_HIP, std::string("glimp_scene_create: ") + hipGetErrorString(e));

@@ -140,16 +140,15 @@ __device__ void diff_pixel(const DiffParams& p, const PixelSlot& ps, PixelState&
         uint32_t tri;
         decode_surface(key, VW.draws, VW.num_draws, S.mi, tri);
         S.tri = tri;
-        const uint8_t* I = p.m.indices + (size_t)S.mi * 384;
-        const float* P = p.m.positions + (size_t)S.mi * 192;
+        const uint32_t corners = p.m.triangles[(size_t)S.mi * 128 + tri];
         float c[3][4], uv[3][2];
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            const uint32_t vi = I[k * 128 + tri];
+            const uint32_t vi = (corners >> (8 * k)) & 255u;
             S.vi[k] = vi;
-            const float px = P[vi], py = P[64 + vi], pz = P[128 + vi];
+            const float4 v = p.m.vertices[(size_t)S.mi * 64 + vi];
 #pragma unroll
-            for (int j = 0; j < 4; j++) c[k][j] = xform(VW.object_to_clip, j, px, py, pz);
+            for (int j = 0; j < 4; j++) c[k][j] = xform(VW.object_to_clip, j, v.x, v.y, v.z);
             const float2 t2 = p.uv[(size_t)S.mi * 64 + vi];
             uv[k][0] = t2.x;
             uv[k][1] = t2.y;
@@ -555,9 +554,11 @@ __global__ void __launch_bounds__(256) k_diff_vertices(DiffParams p, float4* gra
             for (uint32_t i = tid; i < 384; i += 256) s_corner[i / 6][(i / 2) % 3][i & 1] = 0ull;
             __syncthreads();
             const uint32_t nt = min((uint32_t)p.m.num_triangles[mi], 128u);
-            for (uint32_t i = tid; i < 384; i += 256) {
-                const uint32_t k = i >> 7, q = i & 127u, v = p.m.indices[(size_t)mi * 384 + i];
-                if (q < nt && v < 64) atomicOr(&s_corner[v][k][q >> 6], 1ull << (q & 63u));
+            if (tid < nt) {
+                const uint32_t corners = p.m.triangles[(size_t)mi * 128 + tid];
+#pragma unroll
+                for (uint32_t k = 0; k < 3; k++)
+                    atomicOr(&s_corner[(corners >> (8 * k)) & 63u][k][tid >> 6], 1ull << (tid & 63u));
             }
         }
         for (uint32_t g0 = c_lo; g0 < c_hi; g0 += kPartBlocks) {

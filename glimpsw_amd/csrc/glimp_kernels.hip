@@ -2601,15 +2601,16 @@ __device__ __forceinline__ void gbuffer_fragment(const DrawParams& p, const View
     const uint32_t rank = ~keylo;
     const uint32_t prim = ((rank >> 8) & 7u) * 16u + ((rank >> 3) & 15u);
     const uint32_t mi = V.meshlet_offset + ((rank >> 11) - V.seq_base);
-    const uint8_t* I = V.m.indices + (size_t)mi * 384;
+    const uint32_t corners = V.m.triangles[(size_t)mi * 128 + prim];
     float nv[3][3], tv[3][3];
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-        const uint32_t nt = V.m.normal_tangents[(size_t)mi * 64 + (I[q * 128 + prim] & 63u)];
-        unpack_normal(AT, nt, nv[q]);
-        unpack_normal(AT, nt >> 16, tv[q]);
+        const size_t at = (size_t)mi * 64 + ((corners >> (8 * q)) & 255u);
+        const float4 n = V.m.normals[at], t = V.m.tangents[at];
+        nv[q][0] = n.x; nv[q][1] = n.y; nv[q][2] = n.z;
+        tv[q][0] = t.x; tv[q][1] = t.y; tv[q][2] = t.z;
     }
-    const uint32_t handed = (uint32_t)((V.m.tangent_handedness[mi] >> (I[prim] & 63u)) & 1u) << 31;
+    const uint32_t handed = (uint32_t)((V.m.tangent_handedness[mi] >> (corners & 63u)) & 1u) << 31;
     float N[3], Tw[3];
     lerp_to_world(AT, nv, uv.b, V.o2w, N);
     lerp_to_world(AT, tv, uv.b, V.o2w, Tw);
@@ -2866,6 +2867,28 @@ __global__ void k_decode_overdraw(const unsigned long long* counts, const uint32
     if (depth_out) depth_out[o] = depth[i];
 }
 
+// The gather arrays of a scene (DevMeshlets): thread = vertex slot, and two
+// triangle slots.
+__global__ void __launch_bounds__(256) k_expand_meshlets(DevMeshlets m, ApproxTables tables, float4* vertices,
+                                                         float4* normals, float4* tangents, uint32_t* triangles) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (size_t)m.count * 64) return;
+    const size_t mi = i >> 6;
+    const uint32_t v = (uint32_t)(i & 63u);
+    const float* P = m.positions + mi * 192;
+    vertices[i] = make_float4(P[v], P[64 + v], P[128 + v], bitsf(m.texcoords[i]));
+    float n[3], t[3];
+    unpack_normal(tables, m.normal_tangents[i], n);
+    unpack_normal(tables, m.normal_tangents[i] >> 16, t);
+    normals[i] = make_float4(n[0], n[1], n[2], 0.0f);
+    tangents[i] = make_float4(t[0], t[1], t[2], 0.0f);
+    const uint8_t* I = m.indices + mi * 384;
+#pragma unroll
+    for (uint32_t k = v; k < 128; k += 64)
+        triangles[mi * 128 + k] = (uint32_t)(I[k] & 63u) | ((uint32_t)(I[128 + k] & 63u) << 8) |
+                                  ((uint32_t)(I[256 + k] & 63u) << 16);
+}
+
 // The bin raster for the launch's bin size and workgroup size: 128 or 256
 // threads for every bin size, 512 or 1024 for 32- and 64-pixel bins (a
 // crowded large bin then has more waves to spread its tiles over).
@@ -2964,6 +2987,14 @@ void warm_launch_shapes() {
 
 hipError_t launch_reset_counters(DrawScratch* scratch, hipStream_t s) {
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, s, scratch);
+    return hipGetLastError();
+}
+
+hipError_t launch_expand_meshlets(const DevMeshlets& m, const ApproxTables& tables, hipStream_t s) {
+    if (!m.count) return hipSuccess;
+    hipLaunchKernelGGL(k_expand_meshlets, dim3((m.count + 3) / 4), dim3(256), 0, s, m, tables,
+                       const_cast<float4*>(m.vertices), const_cast<float4*>(m.normals),
+                       const_cast<float4*>(m.tangents), const_cast<uint32_t*>(m.triangles));
     return hipGetLastError();
 }
 

@@ -22,6 +22,14 @@ struct DevMeshlets {
     const uint32_t* texcoords;     // [M][64]
     const uint32_t* normal_tangents;
     const uint8_t* indices;        // [M][3][128]
+    // The same for the passes that gather single triangles (resolve, G-buffer,
+    // differentiable resolve), derived once when the scene is created
+    // (launch_expand_meshlets): one 16-byte load per vertex instead of four,
+    // normals already unpacked.
+    const float4* vertices;        // [M][64] position, texcoord bits
+    const float4* normals;         // [M][64] unit vertex normal, 0
+    const float4* tangents;        // [M][64] unit vertex tangent, 0
+    const uint32_t* triangles;     // [M][128] v0 | v1 << 8 | v2 << 16, each below 64
 };
 
 // Per material: face culling and fragment entry point as ShadeMeshlet
@@ -267,6 +275,8 @@ struct DrawParams {
 // process on the device, outside any stream capture).
 void warm_launch_shapes();
 hipError_t launch_draw_direct(const DrawParams& p, hipStream_t s, Profiler* prof);
+// Fills m's gather arrays from its uploaded ones.
+hipError_t launch_expand_meshlets(const DevMeshlets& m, const ApproxTables& tables, hipStream_t s);
 hipError_t launch_draw_binned(const DrawParams& p, hipStream_t s, Profiler* prof);
 // The overdraw pipeline (FS_Overdraw): per pixel the keys hold the covered
 // count in the high and the quad-helper count in the low 32 bits, and
