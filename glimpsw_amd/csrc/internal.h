@@ -142,9 +142,10 @@ constexpr uint32_t kFinePairs = 64;
 constexpr uint32_t kCoarsePairs = 64;
 
 // Per-draw scratch counters, cleared without a launch of their own:
-// num_visible is zero when a draw starts (allocation clears it, the bin
-// raster clears it after its last reader, a direct draw ends with a reset),
-// and the cull clears the others, which only later stages fill.
+// num_visible, num_clip and num_clip_overflow are zero when a draw starts
+// (allocation clears them, the bin raster clears them after their last
+// readers, a direct draw ends with a reset); the draw's first kernel clears
+// the others, which only later stages fill.
 struct DrawScratch {
     uint32_t num_records;          // records appended by the clipper
     uint32_t num_clip;

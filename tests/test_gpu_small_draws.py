@@ -1,0 +1,41 @@
+"""Draws that are culled and set up in one kernel (as many meshlets as there
+are resident waves, or fewer) and draws that are not, one after another on one
+context: ids, depth and counters equal the oracle's bit for bit, so each kind
+leaves the shared counters as the other expects them. Some meshlets surround
+the eye, so triangles are clipped, and some lie outside the view."""
+import numpy as np
+import pytest
+
+import oracle
+from glimpsw_amd import scene as S
+from tests import scenes as T
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("pipeline", ["visibility", "direct"])
+@pytest.mark.parametrize("alpha", [False, True])
+def test_draw_sizes_in_turn(gpu_ctx, alpha, pipeline):
+    import glimpsw_amd as g
+
+    W, H = 320, 240
+    make = T.alpha_scene if alpha else T.small_scene
+    sc = make(9000, seed_offset=11, spread=6.0, near_frac=0.05)
+    ds = g.Scene(gpu_ctx, sc)
+    fb = g.Framebuffer(gpu_ctx, W, H)
+    flags = g.GLIMP_DRAW_COUNTERS | (g.GLIMP_DRAW_DIRECT if pipeline == "direct" else 0)
+    for n in (1, 5, 300, 9000, 63, 64, 5119, 5121, 9000, 2, 4096):
+        view = S.make_view(W, H, count=n)
+        ofb, octr, _ = oracle.render_frame(sc, view)
+        gpu_ctx.reset_counters()
+        fb.clear(0, 0.0)
+        fb.draw(ds, view.object_to_clip, n, 0, view.frustum_planes(), flags)
+        ids, depth = fb.read()
+        ctr = gpu_ctx.counters()
+        print(f"[draws] {n} meshlets: {ctr['triangles_clipped']} clipped", flush=True)
+        assert (ids == ofb.ids()).all()
+        assert (depth.view(np.uint32) == ofb.depth().view(np.uint32)).all()
+        for k in ("triangles_processed", "triangles_rasterized", "triangles_clipped"):
+            assert ctr[k] == octr[k], k
+    fb.close()
+    ds.close()
