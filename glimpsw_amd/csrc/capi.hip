@@ -700,6 +700,18 @@ struct LaunchShape {
     uint32_t raster_threads = 256;
 };
 
+// Bin capacity of a draw that names none: the lists of all its bins take
+// about 16 MiB where that is more than 1,024 entries each, so a small frame
+// of many meshlets keeps its records in the lists. What is past the capacity
+// goes to the overflow pass, where a wave walks each triangle over the whole
+// frame: 10,331 meshlets at 180x156 (120 bins, 3,600 entries each on average)
+// took 457 us with 1,024 entries a bin, 345 of it the overflow, and take 180.
+uint32_t default_bin_capacity(uint64_t bins, uint64_t meshlets) {
+    constexpr uint64_t kEntries = 1ull << 22;
+    const uint64_t room = kEntries / std::max<uint64_t>(bins, 1) / 64 * 64;
+    return (uint32_t)std::max<uint64_t>(LaunchShape().bin_capacity, std::min(room, meshlets * 128));
+}
+
 // Clipped triangles are rare (the reference measures < 0.1%, README.md:93);
 // the clip queue holds up to two per meshlet and every queued triangle may
 // produce 8 fan triangles. What a full queue drops is counted in the
@@ -934,6 +946,7 @@ int glimp_draw_meshlets(glimp_context* c, glimp_framebuffer* f, glimp_scene* s, 
               d->occlusion ? &occ : nullptr);
     const BinTotals bins = direct ? BinTotals() : layout_bins(views, sh.bin_size);
     const bool alpha = (s->has_alpha && !overdraw) || deferred;    // FS_Overdraw has no alpha test
+    if (layers || !d->bin_capacity) sh.bin_capacity = default_bin_capacity(bins.bins, d->meshlet_count);
     const size_t clipq = clip_capacity_for(d->meshlet_count);
     int rc = prepare_scratch(c->draw_scratch, d->meshlet_count, clipq, bins, sh, !direct, alpha);
     if (rc != GLIMP_OK) return rc;

@@ -39,3 +39,26 @@ def test_draw_sizes_in_turn(gpu_ctx, alpha, pipeline):
             assert ctr[k] == octr[k], k
     fb.close()
     ds.close()
+
+
+@pytest.mark.parametrize("size,meshlets", [((16, 16), 3000), ((64, 48), 9000), ((180, 156), 1), ((180, 156), 9000)])
+def test_default_list_capacity(gpu_ctx, size, meshlets):
+    """Small frames of many meshlets: thousands of records in a bin, drawn
+    with the default list capacity and with one that overflows."""
+    import glimpsw_amd as g
+
+    W, H = size
+    sc = T.small_scene(meshlets, seed_offset=12, spread=6.0, near_frac=0.02)
+    view = S.make_view(W, H, count=meshlets)
+    ofb, _, _ = oracle.render_frame(sc, view)
+    ds = g.Scene(gpu_ctx, sc)
+    fb = g.Framebuffer(gpu_ctx, W, H)
+    for cap in (0, 128):
+        print(f"[draws] {W}x{H}, {meshlets} meshlets, capacity {cap}", flush=True)
+        fb.clear(0, 0.0)
+        fb.draw(ds, view.object_to_clip, meshlets, 0, view.frustum_planes(), 0, bin_capacity=cap)
+        ids, depth = fb.read()
+        assert (ids == ofb.ids()).all()
+        assert (depth.view(np.uint32) == ofb.depth().view(np.uint32)).all()
+    fb.close()
+    ds.close()
