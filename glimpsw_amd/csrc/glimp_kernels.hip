@@ -2032,7 +2032,12 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
     // flagged the bins they reached
     const bool merge = flagged != 0;
     if (bin == 0 && tid == 0) clear_setup_counters(p);
-    if (tid == 0 && flagged) p.bin_flags[bin] = 0u;
+    if (merge) {
+        // cleared for the next draw once every wave has read it: a wave that
+        // read the cleared flag would leave its pixels' spill keys behind
+        __syncthreads();
+        if (tid == 0) p.bin_flags[bin] = 0u;
+    }
     if (n == 0 && !merge && !V.fresh) return;  // uniform across the block
     const int hw = V.width / 2, hh = V.height / 2;
     // view fields the tile loop needs, in registers: the compiler does not
