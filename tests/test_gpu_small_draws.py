@@ -62,3 +62,29 @@ def test_default_list_capacity(gpu_ctx, size, meshlets):
         assert (depth.view(np.uint32) == ofb.depth().view(np.uint32)).all()
     fb.close()
     ds.close()
+
+
+@pytest.mark.parametrize("meshlets", [8, 640, 641, 1280, 1281, 2560, 2561])
+def test_split_meshlets(gpu_ctx, meshlets):
+    """Meshlets binned in eight parts and fewer, with ragged record counts and
+    with triangles of one pixel to the whole frame."""
+    import glimpsw_amd as g
+
+    W, H = 644, 360
+    sc = T.ragged(T.small_scene(meshlets, seed_offset=13, spread=8.0, near_frac=0.1))
+    view = S.make_view(W, H, count=meshlets)
+    ofb, octr, _ = oracle.render_frame(sc, view)
+    ds = g.Scene(gpu_ctx, sc)
+    fb = g.Framebuffer(gpu_ctx, W, H)
+    for cap in (0, 3):
+        print(f"[draws] {meshlets} meshlets, capacity {cap}", flush=True)
+        gpu_ctx.reset_counters()
+        fb.clear(0, 0.0)
+        fb.draw(ds, view.object_to_clip, meshlets, 0, view.frustum_planes(), g.GLIMP_DRAW_COUNTERS, bin_capacity=cap)
+        ids, depth = fb.read()
+        ctr = gpu_ctx.counters()
+        assert (ids == ofb.ids()).all()
+        assert (depth.view(np.uint32) == ofb.depth().view(np.uint32)).all()
+        assert ctr["fragments_covered"] == octr["fragments_covered"] and ctr["dropped"] == 0
+    fb.close()
+    ds.close()
