@@ -2076,7 +2076,7 @@ template <int BS, int kThreads, bool Alpha>
 __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long (&keys)[BS * BS],
                            BinTri<BS> (&tl)[kThreads], TileMask<BS> (&tmasks)[bin_masks(BS, kThreads)],
                            uint32_t (&s_wave_total)[kThreads / kWave],
-                           uint32_t (&talpha)[Alpha ? kThreads : 1]) {
+                           uint32_t (&talpha)[Alpha ? kThreads : 1], const ApproxTables& approx) {
     constexpr int kWaves = kThreads / kWave;
     constexpr int kGroups = kThreads / 16;
     const uint32_t vidx = view_of_bin(p, bin);
@@ -2230,7 +2230,7 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
                                                    __builtin_fmaf((float)(int32_t)w2, T.z20, T.z0));
                 bool pass = cov && depth > clearDepth;
                 if (ai != 0xFFFFFFFFu && (__ballot(pass) & (0xFFFFull << (lane & 48u)))) {
-                    const bool ok = alpha_test_tile(p.tables, p.alpha[ai], ((T.keylo >> 7) & 1u) == 0,
+                    const bool ok = alpha_test_tile(approx, p.alpha[ai], ((T.keylo >> 7) & 1u) == 0,
                                                     V.textures, (int32_t)w1, (int32_t)w2, lane);
                     pass = pass && ok;
                 }
@@ -2490,11 +2490,18 @@ __global__ void __launch_bounds__(kThreads) k_bin_raster(DrawParams p) {
     __shared__ TileMask<BS> tmasks[bin_masks(BS, kThreads)];
     __shared__ uint32_t s_wave_total[kThreads / kWave];
     __shared__ uint32_t talpha[Alpha ? kThreads : 1];
+    // the alpha test's reciprocals from LDS (2044x1412 with cutouts: 118.4 ->
+    // 114.8 us), where the table costs no resident block
+    constexpr bool kTables = Alpha && BS <= 16;
+    __shared__ uint2 s_pwl[kTables ? 128 : 1];
     __shared__ uint32_t s_bin;
     if (threadIdx.x == 0) s_bin = ordered_bin(p, blockIdx.x);
+    if constexpr (kTables)
+        for (uint32_t i = threadIdx.x; i < 128; i += kThreads) s_pwl[i] = p.tables.pwl[i];
     __syncthreads();
     // wave-uniform: the bin's corners, its view and list addresses are scalars
-    raster_bin<BS, kThreads, Alpha>(p, (uint32_t)__builtin_amdgcn_readfirstlane((int)s_bin), keys, tl, tmasks, s_wave_total, talpha);
+    raster_bin<BS, kThreads, Alpha>(p, (uint32_t)__builtin_amdgcn_readfirstlane((int)s_bin), keys, tl, tmasks,
+                                    s_wave_total, talpha, kTables ? ApproxTables{ s_pwl } : p.tables);
 }
 
 // ---------------------------------------------------------------- layer pipelines
@@ -2823,10 +2830,9 @@ __device__ __forceinline__ uint32_t gbuffer_pack(const ApproxTables& T, const fl
 // Base colour and layer-2 word of the fragments of one tile of record `ai`
 // (all 16 lanes call it: derivatives and the filter choice span the tile;
 // `match` lanes get theirs).
-__device__ __forceinline__ void gbuffer_fragment(const DrawParams& p, const ViewParams& V, uint32_t ai,
-                                                 uint32_t keylo, int32_t w1, int32_t w2, bool match, uint32_t lane,
+__device__ __forceinline__ void gbuffer_fragment(const DrawParams& p, const ApproxTables& AT, const ViewParams& V,
+                                                 uint32_t ai, uint32_t keylo, int32_t w1, int32_t w2, bool match, uint32_t lane,
                                                  uint32_t& color, uint32_t& ch2) {
-    const ApproxTables& AT = p.tables;
     const AlphaRecord& A = p.alpha[ai];
     const DevTexture& tex = V.textures[A.tex & 0xFFFFFFu];
     const TileUV uv = tile_uv(AT, A, ((keylo >> 7) & 1u) == 0, tex, w1, w2, lane);
@@ -2882,9 +2888,12 @@ __global__ void __launch_bounds__(kThreads) k_bin_gbuffer(DrawParams p) {
     __shared__ unsigned long long keys[BS * BS];
     __shared__ uint32_t color[BS * BS], layer2[BS * BS];
     __shared__ uint8_t won[BS * BS];
+    __shared__ uint2 s_pwl[128];
     __shared__ uint32_t s_bin;
     if (threadIdx.x == 0) s_bin = ordered_bin(p, blockIdx.x);
+    for (uint32_t i = threadIdx.x; i < 128; i += kThreads) s_pwl[i] = p.tables.pwl[i];
     __syncthreads();
+    const ApproxTables approx{ s_pwl };
     const ViewParams& V = p.view;
     const LayerBin b = layer_bin(p, V, s_bin, BS);
     const uint32_t tid = threadIdx.x, lane = lane_id();
@@ -2906,7 +2915,7 @@ __global__ void __launch_bounds__(kThreads) k_bin_gbuffer(DrawParams p) {
                            keys[li] == (((unsigned long long)fbits(depth) << 32) | T.keylo);
         if (!(__ballot(match) & groupMask)) return;
         uint32_t c, ch2;
-        gbuffer_fragment(p, V, sm.record[k], T.keylo, w1, w2, match, lane, c, ch2);
+        gbuffer_fragment(p, approx, V, sm.record[k], T.keylo, w1, w2, match, lane, c, ch2);
         if (match) {
             color[li] = c;
             layer2[li] = ch2;
@@ -3000,7 +3009,7 @@ __global__ void __launch_bounds__(256) k_gbuffer(DrawParams p) {
             if (ai == 0xFFFFFFFFu) continue;
             const ViewParams& V = view_of(p, tview[wid][k]);
             uint32_t color, ch2;
-            gbuffer_fragment(p, V, ai, tl[wid][k].keylo, w1, w2, match, lane, color, ch2);
+            gbuffer_fragment(p, p.tables, V, ai, tl[wid][k].keylo, w1, w2, match, lane, color, ch2);
             if (match) {
                 V.aux[off] = color;
                 V.aux[(size_t)V.width * V.height + off] = ch2;
