@@ -3,11 +3,12 @@
 // One launch per stage covers every view of a draw or batch (a single
 // DrawMeshlets call is a batch of one view, Rasterizer::DrawMeshlets,
 // Rasterizer.h:213):
-//   k_begin       zero the per-launch counters and bin counts
-//   k_cull        frustum test of bound spheres, one lane per meshlet
+//   k_cull        frustum and occlusion test of bound spheres, one lane per
+//                 meshlet
 //   k_mesh_setup  one wave per meshlet: vertex transform into LDS, outcodes,
 //                 triangle setup; survivors become 32-byte TriRecords in the
 //                 meshlet's own slots, guard-band cases go to a clip queue
+//   k_cull_setup  both in one launch, for small draws
 //   k_clip        one wave per queued triangle: wave-parallel
 //                 Sutherland-Hodgman, fan triangulation, setup
 //   k_bin_scatter (record, screen bin) pairs into fixed-capacity bins; a
@@ -1067,21 +1068,18 @@ __global__ void __launch_bounds__(256) k_clip(DrawParams p) {
 // ---------------------------------------------------------------- record chunks
 
 // Chunks of up to 64 records for a wave: chunk c < 2*num_visible is half
-// c&1 of visible meshlet slot c>>1; later chunks cover the clipped records.
+// c&1 of meshlet slot c>>1; later chunks cover the clipped records.
 struct Chunk {
     uint32_t base, count;
-    const uint32_t* list;      // non-null: record index = list[base + i]
 };
 
-__device__ __forceinline__ uint32_t num_chunks(const DrawParams& p, bool with_clipped = true) {
-    if (!with_clipped) return 2 * p.scratch->num_visible;
+__device__ __forceinline__ uint32_t num_chunks(const DrawParams& p) {
     uint32_t nclip = min(p.scratch->num_records, p.clip_record_capacity);
     return 2 * p.scratch->num_visible + (nclip + 63) / 64;
 }
 
 __device__ __forceinline__ Chunk get_chunk(const DrawParams& p, uint32_t c) {
     Chunk k;
-    k.list = nullptr;
     const uint32_t nvis = p.scratch->num_visible;
     if (c < 2 * nvis) {
         uint32_t i = c >> 1, half = c & 1;
@@ -1350,7 +1348,7 @@ __global__ void __launch_bounds__(256) k_raster_direct(DrawParams p) {
         uint32_t ntiles = 0;
         TriLds t;
         if (lane < ck.count) {
-            const uint32_t r = ck.list ? ck.list[ck.base + lane] : ck.base + lane;
+            const uint32_t r = ck.base + lane;
             const TriRecord rec = p.records[r];
             const uint32_t v = rec.flags >> 16;
             const ViewParams& V = view_of(p, v);
@@ -2640,7 +2638,6 @@ __device__ __forceinline__ Chunk spill_chunk(const DrawParams& p, uint32_t c) {
     Chunk k;
     k.base = c * 64;
     k.count = min(64u, min(p.scratch->num_spill, p.spill_capacity) - c * 64);
-    k.list = p.spill;
     return k;
 }
 
@@ -2727,7 +2724,7 @@ __global__ void __launch_bounds__(256) k_raster_overdraw(DrawParams p) {
         uint32_t ntiles = 0;
         TriLds t;
         if (lane < ck.count) {
-            const uint32_t r = ck.list[ck.base + lane];
+            const uint32_t r = p.spill[ck.base + lane];
             const TriRecord rec = p.records[r];
             const uint32_t v = rec.flags >> 16;
             const ViewParams& V = view_of(p, v);
@@ -2953,7 +2950,7 @@ __global__ void __launch_bounds__(256) k_gbuffer(DrawParams p) {
         uint32_t ntiles = 0;
         TriLds t;
         if (lane < ck.count) {
-            const uint32_t r = ck.list[ck.base + lane];
+            const uint32_t r = p.spill[ck.base + lane];
             const TriRecord rec = p.records[r];
             const uint32_t v = rec.flags >> 16;
             const ViewParams& V = view_of(p, v);
