@@ -41,8 +41,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# Vector-ALU issue rate: 256 CUs x 4 SIMDs, a wave64 VALU instruction occupies
-# a 16-lane SIMD for 4 cycles at the 2.4 GHz peak clock.
+# Vector-ALU issue rate: 256 CUs x 4 SIMDs, one wave64 VALU instruction per
+# four cycles of a 16-lane SIMD at the 2.4 GHz peak clock (part of the
+# instructions issue faster: the lit resolve retires 735 G/s).
 VALU_PEAK_WAVE_INSTS = 256 * 4 * 2.4e9 / 4
 
 
@@ -65,6 +66,8 @@ def algorithmic_bytes(stats: dict) -> dict:
         "cull": 16 * m_all + 8 * m_vis,
         # meshlets in, 32-byte records and 64-byte clip entries out
         "mesh_setup": 8 * m_vis + meshlet_in + 32 * S + 64 * Cq,
+        # both in one kernel (small draws)
+        "cull_setup": 16 * m_all + meshlet_in + 32 * S + 64 * Cq,
         "clip": 64 * Cq,
         # records in, covered fragments update one 8-byte key each
         "raster_direct": 32 * S + 8 * F,
@@ -82,7 +85,8 @@ def algorithmic_bytes(stats: dict) -> dict:
 
 # profiler name -> kernel symbol substring in rocprofv3 output
 KERNEL_SYMBOLS = {
-    "clear": "k_clear(", "cull": "k_cull<", "mesh_setup": "k_mesh_setup<", "clip": "k_clip<",
+    "clear": "k_clear(", "cull": "k_cull<", "mesh_setup": "k_mesh_setup<",
+    "cull_setup": "k_cull_setup<", "clip": "k_clip<",
     "bin_scatter": "k_bin_scatter<", "bin_order": "k_bin_order<", "bin_raster": "k_bin_raster<",
     "resolve_lit": "k_resolve<1>",
 }
@@ -200,8 +204,9 @@ def measure_traffic(shape: dict | None) -> dict | None:
 
 
 def _valu_roofline(traffic, name: str, avg_us) -> dict | None:
-    """The kernel's vector-ALU instructions per launch against the VALU issue
-    rate: the time they need at best, and that time over the measured one."""
+    """The kernel's vector-ALU instructions per launch: their time at one per
+    four cycles and SIMD, and that time over the measured one (above 1 where
+    part of them issues faster)."""
     if not traffic or not avg_us or name not in traffic.get("valu", {}):
         return None
     insts = traffic["valu"][name]
@@ -212,7 +217,7 @@ def _valu_roofline(traffic, name: str, avg_us) -> dict | None:
 
 def host_threads() -> int:
     """Host threads this process may use: the CPUs it is allowed to run on,
-    capped by OMP_NUM_THREADS when that is set (the GPU box grants 16)."""
+    capped by OMP_NUM_THREADS when that is set."""
     n = len(os.sched_getaffinity(0)) if hasattr(os, "sched_getaffinity") else (os.cpu_count() or 1)
     cap = os.environ.get("OMP_NUM_THREADS")
     return max(1, min(n, int(cap))) if cap and cap.isdigit() else n
