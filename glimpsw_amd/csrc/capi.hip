@@ -99,7 +99,7 @@ struct Scratch {
     uint32_t* bin_order = nullptr;
     size_t bin_order_cap = 0;
     size_t bin_lists_cap = 0;
-    uint32_t* coarse_counts = nullptr; // cleared by each launch's cull
+    uint32_t* coarse_counts = nullptr; // cleared by each launch's first kernel
     size_t coarse_counts_cap = 0;
     uint32_t* coarse_lists = nullptr;
     size_t coarse_lists_cap = 0;
@@ -824,8 +824,11 @@ int prepare_scratch(Scratch& S, size_t total_meshlets, size_t clipq, const BinTo
     if (rc == GLIMP_OK && S.bin_flags_cap != old_flags_cap)
         HIP_TRY(hipMemset(S.bin_flags, 0, S.bin_flags_cap * sizeof(uint32_t)));
     if (rc == GLIMP_OK && binned) rc = grow_one(S.bin_lists, S.bin_lists_cap, total_bins * sh.bin_capacity);
+    const size_t old_coarse_cap = S.coarse_counts_cap;
     if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_counts, S.coarse_counts_cap,
                                              std::max<size_t>((size_t)bins.l1 + bins.l2, 1));
+    if (rc == GLIMP_OK && S.coarse_counts_cap != old_coarse_cap)
+        HIP_TRY(hipMemset(S.coarse_counts, 0, S.coarse_counts_cap * sizeof(uint32_t)));
     if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_lists, S.coarse_lists_cap,
                                              bins.l1 * coarse_capacity(sh.bin_capacity, 4, recs) +
                                                  bins.l2 * coarse_capacity(sh.bin_capacity, 16, recs));

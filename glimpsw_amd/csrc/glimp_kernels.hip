@@ -2368,7 +2368,7 @@ __device__ void raster_bin(const DrawParams& p, uint32_t bin, unsigned long long
     }
     // the bin's count, read by every thread before the first barrier of the
     // record loop (count > 0 means the loop ran), is cleared for the next
-    // draw (the cull clears the coarser bins' counts, which 16 or 256 bins read)
+    // draw (its first kernel clears the coarser bins' counts, which 16 or 256 bins read)
     // (a deferred draw's G-buffer pass still reads it)
     if (tid == 0 && count && !(Alpha && p.layers)) p.bin_counts[bin] = 0;
     if (countFrags) {
@@ -3016,9 +3016,15 @@ __global__ void __launch_bounds__(256) k_gbuffer(DrawParams p) {
     }
 }
 
-// Clears every scratch counter: at the end of a direct draw (a binned one
-// clears them in its first and last kernels) and in place of the cull of a
-// launch without meshlets.
+// The first kernel of a launch without meshlets, in place of the cull: the
+// raster reads every bin's lists all the same.
+__global__ void __launch_bounds__(256) k_no_meshlets(DrawParams p) {
+    clear_draw_counters(p);
+    if (blockIdx.x == 0 && threadIdx.x == 0) clear_setup_counters(p);
+}
+
+// Clears every scratch counter, at the end of a direct draw (a binned one
+// clears them in its first and last kernels).
 __global__ void k_reset_counters(DrawScratch* s) {
     s->num_records = 0;
     s->num_clip = 0;
@@ -3175,7 +3181,9 @@ bool launch_bin_raster(const DrawParams& p, hipStream_t s, Profiler* prof) {
 }
 
 void launch_front(const DrawParams& p, hipStream_t s, Profiler* prof, bool separate_clip) {
-    if (!p.total_meshlets) hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(1), 0, s, p.scratch);
+    if (!p.total_meshlets)
+        hipLaunchKernelGGL(k_no_meshlets, dim3(min((p.coarse_total + 255) / 256 + 1, kPersistentBlocks)), dim3(256), 0,
+                           s, p);
     const uint32_t want = (p.total_meshlets + 3) / 4;
     const uint32_t scatter_blocks =
         p.alpha ? resident_blocks<k_bin_scatter<true>, 256>() : resident_blocks<k_bin_scatter<false>, 256>();

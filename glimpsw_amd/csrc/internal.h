@@ -249,7 +249,7 @@ struct DrawParams {
     uint32_t* bin_lists;           // [total_bins][bin_capacity]
     // Records whose box covers many bins are listed once per coarser bin:
     // counts of the views' level-1 bins (coarse_l1 of them), then level 2,
-    // cleared by the cull; their lists (all of level 1, then level 2) hold 4
+    // cleared by the launch's first kernel; their lists (all of level 1, then level 2) hold 4
     // and 16 times bin_capacity, at most every record of the launch.
     uint32_t* coarse_counts;
     uint32_t* coarse_lists;
