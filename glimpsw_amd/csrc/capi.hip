@@ -2,6 +2,8 @@
 // draw/read entry points over the kernels in glimp_kernels.hip.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -180,6 +182,7 @@ struct glimp_context {
     Scratch draw_scratch;              // scratch of single draws
     DiffWorkspace diff_ws;             // differentiable resolve backward
     std::vector<DiffTex> diff_tex;     // last texture table uploaded to d_diff_tex
+    bool diff_overlap = false;         // level0_overlap of it
     DiffTex* d_diff_tex = nullptr;
     size_t d_diff_tex_cap = 0;
     DiffView* d_diff_views = nullptr;
@@ -1686,6 +1689,22 @@ int glimp_resolve(glimp_context* c, glimp_framebuffer* f, glimp_scene* sc, const
 
 namespace {
 
+// Whether two textures share level-0 texels without having the same level 0
+// (offset and both sides): the same texel is then the corner of different
+// bilinear cells. Textures of one range, and distinct ranges, are the rule.
+bool level0_overlap(const std::vector<DiffTex>& tex) {
+    std::vector<std::array<uint64_t, 3>> r;
+    for (const auto& t : tex) r.push_back({ t.level_offset[0], t.width, t.height });
+    std::sort(r.begin(), r.end());
+    r.erase(std::unique(r.begin(), r.end()), r.end());
+    uint64_t end = 0;
+    for (const auto& [offset, w, h] : r) {
+        if (offset < end) return true;
+        end = offset + w * h;
+    }
+    return false;
+}
+
 // Shared set-up of the differentiable resolve calls: parameter arrays and
 // the texture table.
 int diff_common(glimp_context* c, glimp_scene* sc, const glimp_diff_desc* d, hipStream_t s, const std::string& who,
@@ -1725,6 +1744,7 @@ int diff_common(glimp_context* c, glimp_scene* sc, const glimp_diff_desc* d, hip
             HIP_TRY(hipMemcpy(c->d_diff_tex, tex.data(), tex.size() * sizeof(DiffTex), hipMemcpyHostToDevice));
         }
         c->diff_tex = tex;
+        c->diff_overlap = level0_overlap(tex);
     }
     memset(&p, 0, sizeof(p));
     p.m = sc->m;
@@ -1828,8 +1848,8 @@ int diff_backward(glimp_context* c, glimp_scene* sc, const glimp_diff_desc* d, c
         return fail(GLIMP_E_INVALID, who + ": NULL gradient array");
     p.grad_out = (const float4*)grad_out;
     HIP_TRY(diff_workspace_reserve(c->diff_ws, p.total_pixels, p.total_blocks, sc->m.count, count));
-    HIP_TRY(launch_diff_backward(p, c->diff_ws, d->num_texels, (float4*)grad_texels, (float2*)grad_uv,
-                                 (float4*)grad_color, s, &c->prof));
+    HIP_TRY(launch_diff_backward(p, c->diff_ws, d->num_texels, c->diff_overlap, (float4*)grad_texels,
+                                 (float2*)grad_uv, (float4*)grad_color, s, &c->prof));
     return GLIMP_OK;
 }
 

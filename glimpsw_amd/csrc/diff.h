@@ -95,8 +95,10 @@ hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks
 void diff_workspace_release(DiffWorkspace& w);
 hipError_t launch_diff_forward(const DiffParams& p, hipStream_t s, Profiler* prof);
 // grad_texels [num_texels], grad_uv [vertices], grad_color [vertices] are
-// overwritten (zeros where nothing contributes).
-hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_texels, float4* grad_texels,
-                                float2* grad_uv, float4* grad_color, hipStream_t s, Profiler* prof);
+// overwritten (zeros where nothing contributes). `overlapping`: the level-0
+// ranges of two textures overlap and are not the same range.
+hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_texels, bool overlapping,
+                                float4* grad_texels, float2* grad_uv, float4* grad_color, hipStream_t s,
+                                Profiler* prof);
 
 }  // namespace glimp

@@ -340,7 +340,9 @@ int glimp_batch_autotune(glimp_batch* batch, void* stream, glimp_batch_shape* ch
  * texel of the chosen level when minifying, else bilinear at level 0 with
  * texel centres at +0.5 and clamped edges) and Repeat wrap. Uncovered pixels
  * give 0, untextured materials sample 1. Gradients are reduced
- * deterministically (bitwise identical run to run). */
+ * deterministically (bitwise identical run to run). Textures may share
+ * texels; where their level-0 ranges overlap without being the same range
+ * (offset, width and height) a backward call takes about twice as long. */
 #define GLIMP_MAX_DIFF_TEXTURES 256
 
 typedef struct glimp_diff_texture {
