@@ -769,10 +769,11 @@ size_t coarse_capacity(size_t bin_capacity, size_t times, size_t record_slots) {
     return std::min(bin_capacity * times, record_slots);
 }
 
-// Lays out the bins of `views` (ViewParams::bin_base to l2_x). A view gets a
-// coarser level only where a record's box can be over the finer one's limit,
-// so small views cost no coarse lists (the lists add at most half the memory
-// of the fine ones).
+// Lays out the bins of `views` (ViewParams::bin_base to l2_x). Only a view of
+// more than kRectBins bins can have a meshlet that spreads over more of them,
+// whose records may use the coarser levels; smaller views get none. (The
+// coarse lists take a third of the fine ones' memory for a 1920x1080 frame,
+// two thirds for a strip of three bin rows.)
 BinTotals layout_bins(std::vector<ViewParams>& views, uint32_t bin_size) {
     BinTotals t;
     for (auto& V : views) {
@@ -783,12 +784,10 @@ BinTotals layout_bins(std::vector<ViewParams>& views, uint32_t bin_size) {
         V.l1_base = t.l1;
         V.l2_base = t.l2;
         V.l1_x = V.l2_x = 0;
-        if (V.bins_x * V.bins_y <= kFinePairs) continue;
+        if (V.bins_x * V.bins_y <= kRectBins) continue;
         V.l1_x = (V.bins_x + 3) / 4;
-        const uint32_t l1_y = (V.bins_y + 3) / 4;
-        t.l1 += V.l1_x * l1_y;
-        if (V.l1_x * l1_y <= kCoarsePairs) continue;
         V.l2_x = (V.bins_x + 15) / 16;
+        t.l1 += V.l1_x * ((V.bins_y + 3) / 4);
         t.l2 += V.l2_x * ((V.bins_y + 15) / 16);
     }
     return t;

@@ -1462,9 +1462,6 @@ __device__ __forceinline__ uint32_t wave_sort_u32(uint32_t v, uint32_t lane) {
 // each wave expands a chunk of records into their (record, bin) pairs with
 // an exclusive scan and inserts the pairs in parallel, so a triangle
 // spanning many bins costs one pass of the wave, not a serial loop.
-// Bins of the rectangle a meshlet's records cover, up to this many: their
-// pair counts, then their next free slots, live in LDS.
-constexpr uint32_t kRectBins = 1024;
 
 // Bins a lane walks for its own records; a wave with a larger record box
 // walks its pairs in parallel instead (16 here: scatter of a 1080p frame 10.6
@@ -1681,7 +1678,9 @@ __device__ __forceinline__ uint32_t box_bins(uint32_t lo, uint32_t hi) {
 // Inserts records spread over a rectangle of more than kRectBins bins (a
 // large patch near the eye, a clipped triangle), each at the level that
 // keeps its pairs few: the bins of level 1 and 2 are 4x4 and 16x16 bins
-// large, and a bin's raster reads the lists of the three bins it lies in. A
+// large, and a bin's raster reads the lists of the three bins it lies in. (A
+// view with such a rectangle has more than kRectBins bins, hence both
+// levels.) A
 // triangle that covers a 1080p view has 8,160 pairs with 16-pixel bins, 510
 // at level 1 and 40 at level 2 (one wave inserts them 256 at a time, a round
 // trip to memory each). 1080p frame with 512 patches around the eye, 16-pixel
@@ -1705,11 +1704,11 @@ __device__ void bin_levels(const DrawParams& p, bool valid, const TriRecord& rec
     }
     if (counting(p)) entries += (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_add(nb), 63);
     auto up = [](uint32_t v) { return (v >> 2) & 0x3FFF3FFFu; };     // both halves / 4
-    if (nb > kFinePairs && V.l1_x) {
+    if (nb > kFinePairs) {
         lo = up(lo);
         hi = up(hi);
         level = 1;
-        if (box_bins(lo, hi) > kCoarsePairs && V.l2_x) {
+        if (box_bins(lo, hi) > kCoarsePairs) {
             lo = up(lo);
             hi = up(hi);
             level = 2;
@@ -2023,12 +2022,14 @@ struct BinLists {
 
 __device__ __forceinline__ BinLists bin_lists(const DrawParams& p, const ViewParams& V, uint32_t bin, uint32_t bx,
                                               uint32_t by) {
-    // the three counts are loaded side by side (a level the view lacks reads
-    // the first count): one round trip to memory instead of three in a row
-    const uint32_t c1 = V.l1_x ? V.l1_base + (by >> 2) * V.l1_x + (bx >> 2) : 0u;
-    const uint32_t c2 = V.l2_x ? V.l2_base + (by >> 4) * V.l2_x + (bx >> 4) : 0u;
+    // the three counts are loaded side by side (in a view without the coarse
+    // levels, the first count twice): one round trip to memory instead of
+    // three in a row
+    const bool coarse = V.l1_x != 0;
+    const uint32_t c1 = coarse ? V.l1_base + (by >> 2) * V.l1_x + (bx >> 2) : 0u;
+    const uint32_t c2 = coarse ? V.l2_base + (by >> 4) * V.l2_x + (bx >> 4) : 0u;
     uint32_t k0 = p.bin_counts[bin], k1 = p.coarse_counts[c1];
-    uint32_t k2 = p.coarse_counts[V.l2_x ? p.coarse_l1 + c2 : 0u];
+    uint32_t k2 = p.coarse_counts[coarse ? p.coarse_l1 + c2 : 0u];
     k0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)k0);
     k1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)k1);
     k2 = (uint32_t)__builtin_amdgcn_readfirstlane((int)k2);
@@ -2037,9 +2038,9 @@ __device__ __forceinline__ BinLists bin_lists(const DrawParams& p, const ViewPar
     l.fine = p.bin_lists + (size_t)bin * p.bin_capacity;
     l.n0 = min(k0, p.bin_capacity);
     l.l1 = p.coarse_lists + (size_t)c1 * p.l1_capacity;
-    l.n1 = V.l1_x ? min(k1, p.l1_capacity) : 0u;
+    l.n1 = coarse ? min(k1, p.l1_capacity) : 0u;
     l.l2 = p.coarse_lists + (size_t)p.coarse_l1 * p.l1_capacity + (size_t)c2 * p.l2_capacity;
-    l.n2 = V.l2_x ? min(k2, p.l2_capacity) : 0u;
+    l.n2 = coarse ? min(k2, p.l2_capacity) : 0u;
     return l;
 }
 

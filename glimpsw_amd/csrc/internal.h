@@ -135,9 +135,13 @@ constexpr uint32_t kBinBuckets = 16;
 // Bin side of the overdraw and deferred pipelines.
 constexpr uint32_t kLayerBin = 16;
 
-// Bins a record's box may cover before it moves to the coarser bins, in
-// meshlets that spread over too many bins to count them in LDS, and level-1
-// bins before it moves to level 2.
+// Bins of the rectangle a meshlet's records cover, up to this many: their
+// pair counts, then their next free slots, live in LDS.
+constexpr uint32_t kRectBins = 1024;
+
+// In meshlets that spread over more, the bins a record's box may cover before
+// it moves to the coarser bins, and the level-1 bins before it moves to level
+// 2.
 constexpr uint32_t kFinePairs = 64;
 constexpr uint32_t kCoarsePairs = 64;
 
@@ -187,8 +191,8 @@ struct ViewParams {
     uint32_t bin_base;             // first global bin of the view
     uint32_t bins_x, bins_y;
     // Coarser bins, 4x4 (level 1) and 16x16 (level 2) bins large: first bin
-    // of the view in the level's numbering and bins per row; l1_x = 0 for
-    // views of up to 16 bins, l2_x = 0 for those of up to 64 level-1 bins.
+    // of the view in the level's numbering and bins per row; both 0 in views
+    // of up to kRectBins bins, where no record reaches them.
     uint32_t l1_base, l1_x, l2_base, l2_x;
     uint32_t seq_base;             // meshlets drawn into the framebuffer before
     int width, height;
@@ -213,9 +217,10 @@ struct ViewParams {
 // (view v owns slots [meshlet_base, meshlet_base + meshlet_count)), and so
 // are the screen bins (view v owns [bin_base, bin_base + bins_x*bins_y)).
 // Bins are bin_size x bin_size pixel squares (a multiple of the 4x4 tile);
-// each bin holds up to bin_capacity record indices. Records larger than 16
-// bins go to bins of 4x4 bins, the largest to bins of 16x16 bins, and a
-// bin's raster reads all three lists. A record with a pair
+// each bin holds up to bin_capacity record indices. In meshlets spread over
+// more than kRectBins bins, records larger than kFinePairs bins go to bins of
+// 4x4 bins, those larger than kCoarsePairs of these to bins of 16x16 bins,
+// and a bin's raster reads all three lists. A record with a pair
 // that finds its bin full is appended to the overflow list instead (once)
 // and flagged; the overflow raster draws it over its render box into the
 // view's spill_keys, marking the bins it reaches, whose rasters skip it and
@@ -249,8 +254,9 @@ struct DrawParams {
     uint32_t* bin_lists;           // [total_bins][bin_capacity]
     // Records whose box covers many bins are listed once per coarser bin:
     // counts of the views' level-1 bins (coarse_l1 of them), then level 2,
-    // cleared by the launch's first kernel; their lists (all of level 1, then level 2) hold 4
-    // and 16 times bin_capacity, at most every record of the launch.
+    // cleared by the launch's first kernel; their lists (all of level 1, then
+    // level 2) hold 4 and 16 times bin_capacity, at most every record of the
+    // launch.
     uint32_t* coarse_counts;
     uint32_t* coarse_lists;
     uint32_t coarse_l1, coarse_total;
