@@ -1846,7 +1846,7 @@ int diff_backward(glimp_context* c, glimp_scene* sc, const glimp_diff_desc* d, c
     if (!grad_out || !grad_texels || !grad_uv || !grad_color)
         return fail(GLIMP_E_INVALID, who + ": NULL gradient array");
     p.grad_out = (const float4*)grad_out;
-    HIP_TRY(diff_workspace_reserve(c->diff_ws, p.total_pixels, p.total_blocks, sc->m.count, count));
+    HIP_TRY(diff_workspace_reserve(c->diff_ws, p.total_pixels, p.total_blocks, sc->m.count, count, p.cell_blocks));
     HIP_TRY(launch_diff_backward(p, c->diff_ws, d->num_texels, c->diff_overlap, (float4*)grad_texels,
                                  (float2*)grad_uv, (float4*)grad_color, s, &c->prof));
     return GLIMP_OK;

@@ -61,15 +61,16 @@ struct DiffParams {
     uint32_t* cells;               // [views][meshlets][8] a bit per cell of the view the meshlet shows in
     uint32_t* cell_counts;         // [meshlets]
     uint32_t* parts_done;          // [meshlets]
-    uint32_t* part_state;          // marked cells; parts
-    uint4* parts;                  // meshlet, part of it, its parts, its first part's place
-    float* part_sums;              // [parts][6][64]
-    uint32_t max_parts, part_cells, cell_blocks;
+    uint32_t* part_state;          // marked cells; parts; parts of split meshlets
+    uint4* parts;                  // meshlet, part of it, its parts, its first part's sums
+    float* part_sums;              // [parts of split meshlets][6][64]
+    uint32_t part_cells, cell_blocks;
+    bool many_parts;
 };
 
 // Device buffers of one backward pass (owned by the context).
 struct DiffWorkspace {
-    size_t pixels = 0, blocks = 0, meshlets = 0, marks_cap = 0;
+    size_t pixels = 0, blocks = 0, meshlets = 0, marks_cap = 0, parts_cap = 0, sums_cap = 0;
     uint32_t* tex_keys = nullptr;
     float4* tex_recs = nullptr;
     float4* cells = nullptr;       // per run of equal texels, at its first record: three corners, flags and width
@@ -91,7 +92,8 @@ struct DiffWorkspace {
     size_t sort_temp_bytes = 0;
 };
 
-hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks, size_t meshlets, size_t views);
+hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks, size_t meshlets, size_t views,
+                                  uint32_t cell_blocks);
 void diff_workspace_release(DiffWorkspace& w);
 hipError_t launch_diff_forward(const DiffParams& p, hipStream_t s, Profiler* prof);
 // grad_texels [num_texels], grad_uv [vertices], grad_color [vertices] are

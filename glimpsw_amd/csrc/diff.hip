@@ -321,7 +321,7 @@ __global__ void __launch_bounds__(256) k_diff_forward(DiffParams p) {
 
 constexpr uint32_t kBlockRuns = 256;   // most runs of a block of pixels: 64 a wave
 constexpr uint32_t kRunSums = 18;      // 3 corners x (colour, U, V)
-constexpr uint32_t kSplitParts = 32768;                    // most parts beyond one per meshlet
+constexpr uint32_t kSplitParts = 32768;        // most parts beyond one per meshlet
 constexpr uint32_t kPartGrid = 2048;   // 8 blocks a CU
 
 // Texel record flags
@@ -482,22 +482,25 @@ __global__ void __launch_bounds__(256) k_count_cells(DiffParams p) {
     if (threadIdx.x == 0 && s_total) atomicAdd(&p.part_state[0], s_total);
 }
 
-// Cells of a part: about kPartBlocks pixel blocks, more when that would
-// make more than max_parts parts.
+// Cells of a part: about kPartBlocks pixel blocks, more when that could make
+// more than kSplitParts parts beyond one per meshlet (a meshlet of c cells has
+// fewer than c / part_cells of those).
 __device__ __forceinline__ uint32_t part_cells(const DiffParams& p) {
-    const uint32_t room = p.max_parts - p.m.count;      // every meshlet's last part may be a short one
-    return max(p.part_cells, (p.part_state[0] + room - 1) / room);
+    if (!p.many_parts) return p.part_cells;
+    return max(p.part_cells, (p.part_state[0] + kSplitParts - 1) / kSplitParts);
 }
 
 // The parts of every meshlet (one for a meshlet that shows nowhere: it writes
-// zeros); the order of the list does not matter.
+// zeros), those of split meshlets with a place for their sums; the order of
+// the list does not matter.
 __global__ void __launch_bounds__(256) k_list_parts(DiffParams p) {
     const uint32_t mi = blockIdx.x * 256 + threadIdx.x;
     if (mi >= p.m.count) return;
     const uint32_t g = part_cells(p);
     const uint32_t n = max(1u, (p.cell_counts[mi] + g - 1) / g);
     const uint32_t at = atomicAdd(&p.part_state[1], n);
-    for (uint32_t k = 0; k < n; k++) p.parts[at + k] = make_uint4(mi, k, n, at);
+    const uint32_t sums = n > 1 ? atomicAdd(&p.part_state[2], n) : 0u;
+    for (uint32_t k = 0; k < n; k++) p.parts[at + k] = make_uint4(mi, k, n, sums);
 }
 
 // One part a block at a time: the runs of its cells' pixel blocks, 256 blocks
@@ -510,6 +513,9 @@ __global__ void __launch_bounds__(256) k_list_parts(DiffParams p) {
 // triangle comparing every run's.
 constexpr uint32_t kRoundRuns = 128;
 constexpr uint32_t kPartBlocks = 256;
+
+// Cells of a part where they are few enough (part_cells)
+uint32_t part_cells_least(uint32_t cell_blocks) { return std::max(1u, kPartBlocks / cell_blocks); }
 
 __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* s_wave, uint32_t& total) {
     const uint32_t lane = __lane_id(), wid = threadIdx.x >> 6;
@@ -674,7 +680,7 @@ __global__ void __launch_bounds__(256) k_diff_vertices(DiffParams p, float4* gra
         bool write = true;
         if (part.z > 1) {
             // a part of several: the last to finish adds them in order
-            float* mine = p.part_sums + (size_t)item * 384;
+            float* mine = p.part_sums + (size_t)(part.w + part.y) * 384;
             mine[ch * 64 + lane] = g0;
             if (wid < 2) mine[(ch + 1) * 64 + lane] = g1;
             __threadfence();
@@ -697,7 +703,7 @@ __global__ void __launch_bounds__(256) k_diff_vertices(DiffParams p, float4* gra
             if (wid < 2) reinterpret_cast<float2*>(grad_color + vtx)[wid] = make_float2(g0, g1);
             else reinterpret_cast<float*>(grad_uv + vtx)[wid - 2] = g0;
         }
-        __syncthreads();       // s_sum, s_idx, s_last
+        __syncthreads();       // s_sum, s_corner, s_last
     }
 }
 
@@ -939,7 +945,19 @@ hipError_t sum_texels(DiffWorkspace& w, const uint32_t* keys, uint32_t n, uint32
 
 }  // namespace
 
-hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks, size_t meshlets, size_t views) {
+namespace {
+
+// Parts the meshlets can have beyond one each: none where the cells of all
+// views make one part (up to 256x256 pixels), kSplitParts at most.
+uint32_t split_parts(size_t meshlets, size_t views, uint32_t cell_blocks) {
+    const size_t group = part_cells_least(cell_blocks), most = (views * 256 + group - 1) / group - 1;
+    return (uint32_t)std::min<size_t>(meshlets * most, kSplitParts);
+}
+
+}  // namespace
+
+hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks, size_t meshlets, size_t views,
+                                  uint32_t cell_blocks) {
     hipError_t e = hipSuccess;
     // cells, then the counters that start at zero with them
     const size_t marks = views * meshlets * 8 + meshlets + 4;
@@ -952,10 +970,23 @@ hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks
     if (meshlets > w.meshlets) {
         w.meshlets = 0;
         e = grow(w.cell_counts, meshlets);
-        if (e == hipSuccess) e = grow(w.part_list, meshlets + kSplitParts);
-        if (e == hipSuccess) e = grow(w.part_sums, (meshlets + kSplitParts) * 384);
         if (e != hipSuccess) return e;
         w.meshlets = meshlets;
+    }
+    const size_t splits = split_parts(meshlets, views, cell_blocks);
+    if (meshlets + splits > w.parts_cap) {
+        w.parts_cap = 0;
+        e = grow(w.part_list, meshlets + splits);
+        if (e != hipSuccess) return e;
+        w.parts_cap = meshlets + splits;
+    }
+    // parts of split meshlets: each has one more than it counts in `splits`
+    const size_t sums = splits + std::min(splits, meshlets);
+    if (sums > w.sums_cap) {
+        w.sums_cap = 0;
+        e = grow(w.part_sums, sums * 384);
+        if (e != hipSuccess) return e;
+        w.sums_cap = sums;
     }
     if (blocks > w.blocks) {
         w.blocks = 0;
@@ -1022,8 +1053,8 @@ hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_tex
     p.cell_counts = w.cell_counts;
     p.parts = w.part_list;
     p.part_sums = w.part_sums;
-    p.max_parts = p.m.count + kSplitParts;
-    p.part_cells = std::max(1u, kPartBlocks / p.cell_blocks);
+    p.many_parts = split_parts(p.m.count, p.num_views, p.cell_blocks) == kSplitParts;
+    p.part_cells = part_cells_least(p.cell_blocks);
     p.block_runs = w.block_runs;
     p.run_mesh = w.run_mesh;
     p.run_tri = w.run_tri;

@@ -1758,7 +1758,7 @@ __device__ bool bin_meshlet(const DrawParams& p, const bool (&valid)[2], const T
     rhi = ~(uint32_t)__builtin_amdgcn_readlane((int)wave_scan(rhi, 0xFFFFFFFFu, min_u16x2), 63);
     // with every record's box at most kWalkPairs bins each lane walks its
     // own records' pairs (`steps` steps); otherwise the wave walks all pairs
-    // in parallel, 64 at a time
+    // in parallel, 256 at a time
     const uint32_t maxnb = wave_max(big);
     const bool wide = maxnb > kWalkPairs;
     const uint32_t steps = wide ? 0u : maxnb;
