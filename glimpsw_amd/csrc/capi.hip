@@ -709,9 +709,9 @@ struct LaunchShape {
 // goes to the overflow pass, where a wave walks each triangle over the whole
 // frame: 10,331 meshlets at 180x156 (120 bins, 3,600 entries each on average)
 // took 457 us with 1,024 entries a bin, 345 of it the overflow, and take 180.
+constexpr uint64_t kListEntries = 1ull << 22;
 uint32_t default_bin_capacity(uint64_t bins, uint64_t meshlets) {
-    constexpr uint64_t kEntries = 1ull << 22;
-    const uint64_t room = kEntries / std::max<uint64_t>(bins, 1) / 64 * 64;
+    const uint64_t room = kListEntries / std::max<uint64_t>(bins, 1) / 64 * 64;
     return (uint32_t)std::max<uint64_t>(LaunchShape().bin_capacity, std::min(room, meshlets * 128));
 }
 
@@ -769,6 +769,30 @@ size_t coarse_capacity(size_t bin_capacity, size_t times, size_t record_slots) {
     return std::min(bin_capacity * times, record_slots);
 }
 
+// List entries of a draw's bins, and of its coarser bins.
+struct ListEntries {
+    size_t fine = 0, coarse = 0;
+};
+
+ListEntries list_entries(const BinTotals& bins, size_t bin_capacity, size_t record_slots) {
+    return { bins.bins * bin_capacity, bins.l1 * coarse_capacity(bin_capacity, 4, record_slots) +
+                                           bins.l2 * coarse_capacity(bin_capacity, 16, record_slots) };
+}
+
+// Lists to allocate for a draw with the default capacity: what a draw of no
+// more meshlets into any framebuffer no larger in either direction needs, so
+// that after the largest draw none allocates (a stream that is being captured
+// must not). A smaller framebuffer's bins hold more entries each: up to
+// kListEntries in all, and its coarser bins, from kRectBins bins on, no more
+// than that together.
+ListEntries default_list_entries(const BinTotals& bins, size_t bin_capacity, size_t meshlets, size_t record_slots) {
+    ListEntries n = list_entries(bins, bin_capacity, record_slots);
+    n.fine = std::max<size_t>(n.fine, std::min<size_t>(bins.bins * meshlets * 128, kListEntries));
+    const size_t most = list_entries(bins, kListEntries / kRectBins, record_slots).coarse;
+    n.coarse = std::max<size_t>(n.coarse, std::min<size_t>(most, kListEntries));
+    return n;
+}
+
 // Lays out the bins of `views` (ViewParams::bin_base to l2_x). Only a view of
 // more than kRectBins bins can have a meshlet that spreads over more of them,
 // whose records may use the coarser levels; smaller views get none. (The
@@ -807,7 +831,7 @@ uint64_t count_bins(const std::vector<ViewParams>& views, uint32_t bin_size) {
 size_t spill_capacity_for(size_t record_slots) { return record_slots; }
 
 int prepare_scratch(Scratch& S, size_t total_meshlets, size_t clipq, const BinTotals& bins, const LaunchShape& sh,
-                    bool binned, bool alpha) {
+                    bool binned, bool alpha, bool default_capacity) {
     const size_t total_bins = bins.bins;
     const size_t recs = total_meshlets * 128 + clipq * 8;
     int rc = grow_one(S.records, S.records_cap, recs);
@@ -825,15 +849,15 @@ int prepare_scratch(Scratch& S, size_t total_meshlets, size_t clipq, const BinTo
     if (rc == GLIMP_OK && binned) rc = grow_one(S.bin_flags, S.bin_flags_cap, std::max<size_t>(total_bins, 1));
     if (rc == GLIMP_OK && S.bin_flags_cap != old_flags_cap)
         HIP_TRY(hipMemset(S.bin_flags, 0, S.bin_flags_cap * sizeof(uint32_t)));
-    if (rc == GLIMP_OK && binned) rc = grow_one(S.bin_lists, S.bin_lists_cap, total_bins * sh.bin_capacity);
+    const ListEntries lists = default_capacity ? default_list_entries(bins, sh.bin_capacity, total_meshlets, recs)
+                                               : list_entries(bins, sh.bin_capacity, recs);
+    if (rc == GLIMP_OK && binned) rc = grow_one(S.bin_lists, S.bin_lists_cap, lists.fine);
     const size_t old_coarse_cap = S.coarse_counts_cap;
     if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_counts, S.coarse_counts_cap,
                                              std::max<size_t>((size_t)bins.l1 + bins.l2, 1));
     if (rc == GLIMP_OK && S.coarse_counts_cap != old_coarse_cap)
         HIP_TRY(hipMemset(S.coarse_counts, 0, S.coarse_counts_cap * sizeof(uint32_t)));
-    if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_lists, S.coarse_lists_cap,
-                                             bins.l1 * coarse_capacity(sh.bin_capacity, 4, recs) +
-                                                 bins.l2 * coarse_capacity(sh.bin_capacity, 16, recs));
+    if (rc == GLIMP_OK && binned) rc = grow_one(S.coarse_lists, S.coarse_lists_cap, lists.coarse);
     if (rc == GLIMP_OK && binned) rc = grow_one(S.bin_order, S.bin_order_cap, total_bins * kBinBuckets);
     if (rc == GLIMP_OK && binned) rc = grow_one(S.spill, S.spill_cap, spill_capacity_for(recs));
     if (rc == GLIMP_OK && alpha) rc = grow_one(S.alpha, S.alpha_cap, S.records_cap);
@@ -951,9 +975,10 @@ int glimp_draw_meshlets(glimp_context* c, glimp_framebuffer* f, glimp_scene* s, 
               d->occlusion ? &occ : nullptr);
     const BinTotals bins = direct ? BinTotals() : layout_bins(views, sh.bin_size);
     const bool alpha = (s->has_alpha && !overdraw) || deferred;    // FS_Overdraw has no alpha test
-    if (layers || !d->bin_capacity) sh.bin_capacity = default_bin_capacity(bins.bins, d->meshlet_count);
+    const bool default_capacity = layers || !d->bin_capacity;
+    if (default_capacity) sh.bin_capacity = default_bin_capacity(bins.bins, d->meshlet_count);
     const size_t clipq = clip_capacity_for(d->meshlet_count);
-    int rc = prepare_scratch(c->draw_scratch, d->meshlet_count, clipq, bins, sh, !direct, alpha);
+    int rc = prepare_scratch(c->draw_scratch, d->meshlet_count, clipq, bins, sh, !direct, alpha, default_capacity);
     if (rc != GLIMP_OK) return rc;
     DrawParams p;
     memset(&p, 0, sizeof(p));
@@ -1091,8 +1116,8 @@ int layout_batch(glimp_batch* b) {
     b->bins = layout_bins(b->views, b->shape.bin_size);
     b->alpha = false;
     for (const auto& d : b->descs) b->alpha = b->alpha || d.scene->has_alpha;
-    int rc = prepare_scratch(b->scratch, b->total_meshlets, b->clip_triangles, b->bins, b->shape, true,
-                             b->alpha);
+    int rc = prepare_scratch(b->scratch, b->total_meshlets, b->clip_triangles, b->bins, b->shape, true, b->alpha,
+                             false);
     if (rc != GLIMP_OK) return rc;
     if (!b->d_views) HIP_TRY(dev_alloc(&b->d_views, b->views.size()));
     HIP_TRY(hipMemcpy(b->d_views, b->views.data(), b->views.size() * sizeof(ViewParams), hipMemcpyHostToDevice));
