@@ -61,9 +61,9 @@ struct DiffParams {
     uint32_t* cells;               // [views][meshlets][8] a bit per cell of the view the meshlet shows in
     uint32_t* cell_counts;         // [meshlets]
     uint32_t* parts_done;          // [meshlets]
-    uint32_t* part_state;          // marked cells; parts; parts of split meshlets
-    uint4* parts;                  // meshlet, part of it, its parts, its first part's sums
-    float* part_sums;              // [parts of split meshlets][6][64]
+    uint32_t* part_state;          // marked cells; parts
+    uint4* parts;                  // meshlet, part of it, its parts, its first part's place
+    float* part_sums;              // [parts][6][64], where meshlets can have several
     uint32_t part_cells, cell_blocks;
     bool many_parts;
 };
