@@ -709,8 +709,21 @@ struct LaunchShape {
 // goes to the overflow pass, where a wave walks each triangle over the whole
 // frame: 10,331 meshlets at 180x156 (120 bins, 3,600 entries each on average)
 // took 457 us with 1,024 entries a bin, 345 of it the overflow, and take 180.
+// A frame of fewer than kFewBins bins keeps 1,024: its bins' blocks would walk
+// everything while the rest of the card is idle, and the overflow's triangles
+// are small there. 20,000 meshlets of the same density, with 1,024 entries and
+// with longer lists: 1 bin 95 and 820 us, 4 bins 110 and 311, 16 bins 135 and
+// 139, 48 bins 194 and 103; over seven scenes the lines cross between 20 and 36.
+// The overdraw and deferred pipelines (`layers`) walk a bin's list more slowly
+// and their overflow 64 records a wave: in few bins they keep a short list
+// where it would overflow anyway, else the long one. Overdraw of 20,000
+// meshlets in 1 and 16 bins with 64, 1,024 and all entries: 133, 205, 2,847
+// and 369, 452, 561 us; of 3,000: 81, 161, 658 and 313, 173, 173.
 constexpr uint64_t kListEntries = 1ull << 22;
-uint32_t default_bin_capacity(uint64_t bins, uint64_t meshlets) {
+constexpr uint64_t kFewBins = 24;
+uint32_t default_bin_capacity(uint64_t bins, uint64_t meshlets, bool layers) {
+    if (bins < kFewBins && !layers) return LaunchShape().bin_capacity;
+    if (bins < kFewBins && (bins <= 2 || meshlets > 512 * bins)) return 64;
     const uint64_t room = kListEntries / std::max<uint64_t>(bins, 1) / 64 * 64;
     return (uint32_t)std::max<uint64_t>(LaunchShape().bin_capacity, std::min(room, meshlets * 128));
 }
@@ -787,7 +800,8 @@ ListEntries list_entries(const BinTotals& bins, size_t bin_capacity, size_t reco
 // than that together.
 ListEntries default_list_entries(const BinTotals& bins, size_t bin_capacity, size_t meshlets, size_t record_slots) {
     ListEntries n = list_entries(bins, bin_capacity, record_slots);
-    n.fine = std::max<size_t>(n.fine, std::min<size_t>(bins.bins * meshlets * 128, kListEntries));
+    if (bins.bins >= kFewBins)
+        n.fine = std::max<size_t>(n.fine, std::min<size_t>(bins.bins * meshlets * 128, kListEntries));
     const size_t most = list_entries(bins, kListEntries / kRectBins, record_slots).coarse;
     n.coarse = std::max<size_t>(n.coarse, std::min<size_t>(most, kListEntries));
     return n;
@@ -976,7 +990,7 @@ int glimp_draw_meshlets(glimp_context* c, glimp_framebuffer* f, glimp_scene* s, 
     const BinTotals bins = direct ? BinTotals() : layout_bins(views, sh.bin_size);
     const bool alpha = (s->has_alpha && !overdraw) || deferred;    // FS_Overdraw has no alpha test
     const bool default_capacity = layers || !d->bin_capacity;
-    if (default_capacity) sh.bin_capacity = default_bin_capacity(bins.bins, d->meshlet_count);
+    if (default_capacity) sh.bin_capacity = default_bin_capacity(bins.bins, d->meshlet_count, layers);
     const size_t clipq = clip_capacity_for(d->meshlet_count);
     int rc = prepare_scratch(c->draw_scratch, d->meshlet_count, clipq, bins, sh, !direct, alpha, default_capacity);
     if (rc != GLIMP_OK) return rc;
