@@ -1841,7 +1841,10 @@ int diff_setup(glimp_context* c, glimp_scene* sc, const glimp_diff_desc* d, cons
         table[i].blocks_y = ((uint32_t)table[i].height + 15) / 16;
         table[i].cell_w = (table[i].blocks_x + 15) / 16;
         table[i].cell_h = (table[i].blocks_y + 15) / 16;
+        table[i].cells_x = (table[i].blocks_x + table[i].cell_w - 1) / table[i].cell_w;
+        const uint32_t cells_y = (table[i].blocks_y + table[i].cell_h - 1) / table[i].cell_h;
         p.cell_blocks = std::max(p.cell_blocks, table[i].cell_w * table[i].cell_h);
+        p.cell_words = std::max(p.cell_words, (table[i].cells_x * cells_y + 31) / 32);
         blocks += (uint64_t)table[i].blocks_x * table[i].blocks_y;
         if (base >= (1ull << 31)) return fail(GLIMP_E_LIMIT, who + ": more than 2^31 pixels in one call");
     }
@@ -1885,7 +1888,7 @@ int diff_backward(glimp_context* c, glimp_scene* sc, const glimp_diff_desc* d, c
     if (!grad_out || !grad_texels || !grad_uv || !grad_color)
         return fail(GLIMP_E_INVALID, who + ": NULL gradient array");
     p.grad_out = (const float4*)grad_out;
-    HIP_TRY(diff_workspace_reserve(c->diff_ws, p.total_pixels, p.total_blocks, sc->m.count, count, p.cell_blocks));
+    HIP_TRY(diff_workspace_reserve(c->diff_ws, p));
     HIP_TRY(launch_diff_backward(p, c->diff_ws, d->num_texels, c->diff_overlap, (float4*)grad_texels,
                                  (float2*)grad_uv, (float4*)grad_color, s, &c->prof));
     return GLIMP_OK;

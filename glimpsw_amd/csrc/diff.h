@@ -25,7 +25,8 @@ struct DiffView {
     uint32_t num_draws;
     uint32_t pixel_base;
     uint32_t block_base, blocks_x, blocks_y;   // 16x16-pixel blocks of the backward, all views' in one numbering
-    uint32_t cell_w, cell_h;       // blocks per cell of the 16x16 grid over the view
+    uint32_t cell_w, cell_h;       // blocks per cell of the grid of up to 16x16 cells over the view
+    uint32_t cells_x;              // cells per row of it
     float object_to_clip[16];
     float scale_x, scale_y, center_x, center_y, kx, ky;
 };
@@ -58,19 +59,19 @@ struct DiffParams {
     uint8_t* run_same;             // [total_blocks][256] the block's other runs of the meshlet
     float* run_sums;               // [total_blocks][256][18]
     // the vertex gradients' work list
-    uint32_t* cells;               // [views][meshlets][8] a bit per cell of the view the meshlet shows in
+    uint32_t* cells;               // [views][meshlets][cell_words] a bit per cell of the view the meshlet shows in
     uint32_t* cell_counts;         // [meshlets]
     uint32_t* parts_done;          // [meshlets]
     uint32_t* part_state;          // marked cells; parts
     uint4* parts;                  // meshlet, part of it, its parts, its first part's place
     float* part_sums;              // [parts][6][64], where meshlets can have several
-    uint32_t part_cells, cell_blocks;
+    uint32_t part_cells, cell_blocks, cell_words;
     bool many_parts;
 };
 
 // Device buffers of one backward pass (owned by the context).
 struct DiffWorkspace {
-    size_t pixels = 0, blocks = 0, meshlets = 0, marks_cap = 0, parts_cap = 0, sums_cap = 0;
+    size_t pixels = 0, blocks = 0, marks_cap = 0, parts_cap = 0, sums_cap = 0;
     uint32_t* tex_keys = nullptr;
     float4* tex_recs = nullptr;
     float4* cells = nullptr;       // per run of equal texels, at its first record: three corners, flags and width
@@ -79,8 +80,7 @@ struct DiffWorkspace {
     uint8_t* parts = nullptr;      // per 256-record tile the pieces of runs that cross it
     uint2* last = nullptr;         // per tile its last run (texel, first record) when that goes on
     uint32_t* spans = nullptr;
-    uint32_t* marks = nullptr;     // cells, parts_done, part_state
-    uint32_t* cell_counts = nullptr;
+    uint32_t* marks = nullptr;     // cells, cell_counts, parts_done, part_state
     uint4* part_list = nullptr;
     float* part_sums = nullptr;
     uint32_t* block_runs = nullptr;
@@ -92,8 +92,8 @@ struct DiffWorkspace {
     size_t sort_temp_bytes = 0;
 };
 
-hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks, size_t meshlets, size_t views,
-                                  uint32_t cell_blocks);
+// For the calls of p: its views, blocks, cells and scene.
+hipError_t diff_workspace_reserve(DiffWorkspace& w, const DiffParams& p);
 void diff_workspace_release(DiffWorkspace& w);
 hipError_t launch_diff_forward(const DiffParams& p, hipStream_t s, Profiler* prof);
 // grad_texels [num_texels], grad_uv [vertices], grad_color [vertices] are

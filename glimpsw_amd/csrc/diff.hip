@@ -20,7 +20,7 @@
 // Vertices. A block covers 16x16 pixels of one view; each of its waves sums,
 // per triangle it shows (a run), the 18 products of barycentric weight and
 // (dL/dcol, dL/dU, dL/dV) over the run's pixels in lane order, and marks in
-// which cells of a 16x16 grid over the view each of its meshlets shows.
+// which cells of a grid of up to 16x16 over the view each of its meshlets shows.
 // k_diff_vertices walks a meshlet's marked cells in order, adds the meshlet's
 // runs per triangle and then the triangles' corners per vertex; a meshlet of
 // many cells is split into parts, added in order by the last one to finish.
@@ -424,8 +424,8 @@ __global__ void __launch_bounds__(256) k_diff_pixels(DiffParams p) {
         p.run_tri[base + pos] = s_tri[tid];
         // mark the meshlet's cell (a plain read first: nearly every block finds it marked)
         const DiffView& V = view_at(p, ps.view);
-        const uint32_t cell = (by / V.cell_h) * 16 + bx / V.cell_w;
-        uint32_t* word = p.cells + ((size_t)ps.view * p.m.count + mesh) * 8 + (cell >> 5);
+        const uint32_t cell = (by / V.cell_h) * V.cells_x + bx / V.cell_w;
+        uint32_t* word = p.cells + ((size_t)ps.view * p.m.count + mesh) * p.cell_words + (cell >> 5);
         const uint32_t bit = 1u << (cell & 31u);
         if (!(__atomic_load_n(word, __ATOMIC_RELAXED) & bit)) atomicOr(word, bit);
     }
@@ -462,6 +462,10 @@ __global__ void __launch_bounds__(256) k_diff_pixels(DiffParams p) {
 // ---------------------------------------------------------------- backward: vertices
 
 // Marked cells of each meshlet, and of all together (they set the part size).
+// A row of blocks takes about kCountViews of the views (256 views of 16x16
+// pixels, 200 meshlets: one block's loop over all of them took 72 us).
+constexpr uint32_t kCountViews = 32;
+
 __global__ void __launch_bounds__(256) k_count_cells(DiffParams p) {
     __shared__ uint32_t s_total;
     const uint32_t mi = blockIdx.x * 256 + threadIdx.x;
@@ -469,13 +473,17 @@ __global__ void __launch_bounds__(256) k_count_cells(DiffParams p) {
     __syncthreads();
     uint32_t n = 0;
     if (mi < p.m.count) {
-        for (uint32_t v = 0; v < p.num_views; v++) {
-            const uint4* w = reinterpret_cast<const uint4*>(p.cells + ((size_t)v * p.m.count + mi) * 8);
-            const uint4 a = w[0], b = w[1];
-            n += __popc(a.x) + __popc(a.y) + __popc(a.z) + __popc(a.w) + __popc(b.x) + __popc(b.y) + __popc(b.z) +
-                 __popc(b.w);
+        for (uint32_t v = blockIdx.y; v < p.num_views; v += gridDim.y) {
+            const uint32_t* w = p.cells + ((size_t)v * p.m.count + mi) * p.cell_words;
+            if (p.cell_words == 8) {
+                const uint4 a = reinterpret_cast<const uint4*>(w)[0], b = reinterpret_cast<const uint4*>(w)[1];
+                n += __popc(a.x) + __popc(a.y) + __popc(a.z) + __popc(a.w) + __popc(b.x) + __popc(b.y) +
+                     __popc(b.z) + __popc(b.w);
+            } else {
+                for (uint32_t k = 0; k < p.cell_words; k++) n += __popc(w[k]);
+            }
         }
-        p.cell_counts[mi] = n;
+        if (n) atomicAdd(&p.cell_counts[mi], n);
     }
     if (n) atomicAdd(&s_total, n);
     __syncthreads();
@@ -575,13 +583,14 @@ __global__ void __launch_bounds__(256) k_diff_vertices(DiffParams p, float4* gra
             const uint32_t g1 = min(c_hi, g0 + kPartBlocks);
             // cells [g0, g1) of the meshlet's, in (view, cell) order
             uint32_t seen = 0;
-            for (uint32_t v0 = 0; v0 < p.num_views && seen < g1; v0 += 32) {
-                const uint32_t v = v0 + (tid >> 3);
-                uint32_t w = v < p.num_views ? p.cells[((size_t)v * p.m.count + mi) * 8 + (tid & 7u)] : 0u;
+            const uint32_t words = p.num_views * p.cell_words;
+            for (uint32_t w0 = 0; w0 < words && seen < g1; w0 += 256) {
+                const uint32_t v = (w0 + tid) / p.cell_words, k = w0 + tid - v * p.cell_words;
+                uint32_t w = w0 + tid < words ? p.cells[((size_t)v * p.m.count + mi) * p.cell_words + k] : 0u;
                 uint32_t total = 0;
                 uint32_t rank = seen + block_scan((uint32_t)__popc(w), s_wave, total);
                 for (; w && rank < g1; w &= w - 1, rank++)
-                    if (rank >= g0) s_cells[rank - g0] = (v << 8) | (tid & 7u) * 32 + (uint32_t)__builtin_ctz(w);
+                    if (rank >= g0) s_cells[rank - g0] = (v << 8) | (k * 32 + (uint32_t)__builtin_ctz(w));
                 seen += total;
             }
             __syncthreads();
@@ -595,7 +604,8 @@ __global__ void __launch_bounds__(256) k_diff_vertices(DiffParams p, float4* gra
                     const uint32_t vc = s_cells[i];
                     const DiffView& V = view_at(p, vc >> 8);
                     const uint32_t dy = q / V.cell_w, dx = q - dy * V.cell_w;
-                    const uint32_t x = (vc & 15u) * V.cell_w + dx, y = ((vc >> 4) & 15u) * V.cell_h + dy;
+                    const uint32_t cy = (vc & 255u) / V.cells_x, cx = (vc & 255u) - cy * V.cells_x;
+                    const uint32_t x = cx * V.cell_w + dx, y = cy * V.cell_h + dy;
                     if (dy < V.cell_h && x < V.blocks_x && y < V.blocks_y) {
                         const uint32_t b = V.block_base + y * V.blocks_x + x;
                         base = (size_t)b * kBlockRuns;
@@ -950,31 +960,29 @@ namespace {
 
 // Parts the meshlets can have beyond one each: none where the cells of all
 // views make one part (up to 256x256 pixels), kSplitParts at most.
-uint32_t split_parts(size_t meshlets, size_t views, uint32_t cell_blocks) {
-    const size_t group = part_cells_least(cell_blocks), most = (views * 256 + group - 1) / group - 1;
-    return (uint32_t)std::min<size_t>(meshlets * most, kSplitParts);
+uint32_t split_parts(const DiffParams& p) {
+    const size_t group = part_cells_least(p.cell_blocks), cells = (size_t)p.num_views * p.cell_words * 32;
+    return (uint32_t)std::min<size_t>(p.m.count * ((cells + group - 1) / group - 1), kSplitParts);
 }
+
+size_t cell_mark_words(const DiffParams& p) { return (size_t)p.num_views * p.m.count * p.cell_words; }
+
+// The marks with the counters that start at zero beside them
+size_t zeroed_words(const DiffParams& p) { return cell_mark_words(p) + 2 * (size_t)p.m.count + 4; }
 
 }  // namespace
 
-hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks, size_t meshlets, size_t views,
-                                  uint32_t cell_blocks) {
+hipError_t diff_workspace_reserve(DiffWorkspace& w, const DiffParams& p) {
+    const size_t pixels = p.total_pixels, blocks = p.total_blocks, meshlets = p.m.count;
     hipError_t e = hipSuccess;
-    // cells, then the counters that start at zero with them
-    const size_t marks = views * meshlets * 8 + meshlets + 4;
+    const size_t marks = zeroed_words(p);
     if (marks > w.marks_cap) {
         w.marks_cap = 0;
         e = grow(w.marks, marks);
         if (e != hipSuccess) return e;
         w.marks_cap = marks;
     }
-    if (meshlets > w.meshlets) {
-        w.meshlets = 0;
-        e = grow(w.cell_counts, meshlets);
-        if (e != hipSuccess) return e;
-        w.meshlets = meshlets;
-    }
-    const size_t splits = split_parts(meshlets, views, cell_blocks);
+    const size_t splits = split_parts(p);
     if (meshlets + splits > w.parts_cap) {
         w.parts_cap = 0;
         e = grow(w.part_list, meshlets + splits);
@@ -1027,7 +1035,7 @@ hipError_t diff_workspace_reserve(DiffWorkspace& w, size_t pixels, size_t blocks
 void diff_workspace_release(DiffWorkspace& w) {
     void* ptrs[] = { w.tex_keys, w.tex_recs, w.cells, w.sorted_keys, w.sorted_idx, w.parts,
                      w.last,     w.spans,    w.marks, w.block_runs,  w.run_mesh,   w.run_tri, w.run_same, w.run_sums, w.sort_temp,
-                     w.cell_counts, w.part_list, w.part_sums };
+                     w.part_list, w.part_sums };
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     w = DiffWorkspace();
@@ -1046,14 +1054,13 @@ hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_tex
     p.tex_keys = w.tex_keys;
     p.tex_recs = w.tex_recs;
     p.tex_sentinel = (uint32_t)num_texels;
-    const size_t cell_words = (size_t)p.num_views * p.m.count * 8;
     p.cells = w.marks;
-    p.parts_done = w.marks + cell_words;
+    p.cell_counts = w.marks + cell_mark_words(p);
+    p.parts_done = p.cell_counts + p.m.count;
     p.part_state = p.parts_done + p.m.count;
-    p.cell_counts = w.cell_counts;
     p.parts = w.part_list;
     p.part_sums = w.part_sums;
-    p.many_parts = split_parts(p.m.count, p.num_views, p.cell_blocks) == kSplitParts;
+    p.many_parts = split_parts(p) == kSplitParts;
     p.part_cells = part_cells_least(p.cell_blocks);
     p.block_runs = w.block_runs;
     p.run_mesh = w.run_mesh;
@@ -1065,7 +1072,7 @@ hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_tex
         Profiler::Scope sc(prof, "diff_zero_grads", s);
         e = fill_zero(grad_texels, num_texels * 4, s);
         if (e != hipSuccess) return e;
-        const size_t words = cell_words + p.m.count + 4;
+        const size_t words = zeroed_words(p);
         hipLaunchKernelGGL(k_fill_u32, dim3((uint32_t)std::min<size_t>((words + 255) / 256, 4096)), dim3(256), 0, s,
                            w.marks, words, 0u);
         e = hipGetLastError();
@@ -1074,7 +1081,8 @@ hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_tex
     launch_kernel(prof, "diff_pixels", k_diff_pixels, dim3(p.total_blocks), dim3(256), 0, s, p);
     if (p.m.count) {
         const uint32_t mb = (p.m.count + 255) / 256;
-        launch_kernel(prof, "diff_cells", k_count_cells, dim3(mb), dim3(256), 0, s, p);
+        const uint32_t rows = std::min((p.num_views + kCountViews - 1) / kCountViews, 1024u);
+        launch_kernel(prof, "diff_cells", k_count_cells, dim3(mb, rows), dim3(256), 0, s, p);
         launch_kernel(prof, "diff_parts", k_list_parts, dim3(mb), dim3(256), 0, s, p);
         launch_kernel(prof, "diff_vertices", k_diff_vertices, dim3(kPartGrid), dim3(256), 0, s, p, grad_color, grad_uv);
     }
