@@ -65,7 +65,7 @@ struct DiffParams {
     uint32_t* part_state;          // marked cells; parts
     uint4* parts;                  // meshlet, part of it, its parts, its first part's place
     float* part_sums;              // [parts][6][64], where meshlets can have several
-    uint32_t part_cells, cell_blocks, cell_words;
+    uint32_t part_cells, part_cells_least, cell_blocks, cell_words;
     bool many_parts;
 };
 

@@ -323,6 +323,7 @@ constexpr uint32_t kBlockRuns = 256;   // most runs of a block of pixels: 64 a w
 constexpr uint32_t kRunSums = 18;      // 3 corners x (colour, U, V)
 constexpr uint32_t kSplitParts = 32768;        // most parts beyond one per meshlet
 constexpr uint32_t kPartGrid = 2048;   // 8 blocks a CU
+constexpr uint32_t kFillParts = 1024;
 
 // Texel record flags
 constexpr uint32_t kTexLinear = 1u, kTexRight = 2u, kTexBelow = 4u;
@@ -490,12 +491,17 @@ __global__ void __launch_bounds__(256) k_count_cells(DiffParams p) {
     if (threadIdx.x == 0 && s_total) atomicAdd(&p.part_state[0], s_total);
 }
 
-// Cells of a part: about kPartBlocks pixel blocks, more when that could make
-// more than kSplitParts parts beyond one per meshlet (a meshlet of c cells has
-// fewer than c / part_cells of those).
+// Cells of a part: about kPartBlocks pixel blocks; in scenes of fewer than
+// kFillParts meshlets down to a quarter of that, for kFillParts parts; more
+// when it could make more than kSplitParts beyond one per meshlet (a meshlet
+// of c cells has fewer than c / part_cells of those). 256 views of 16x16
+// pixels, 200 meshlets: whole parts 361 us, quarters 274; one 704x512 view,
+// 500 meshlets 283 and 236. With 6,000 meshlets the card is full as it is:
+// quarters made three 1280x720 views 797 us instead of 732.
 __device__ __forceinline__ uint32_t part_cells(const DiffParams& p) {
-    if (!p.many_parts) return p.part_cells;
-    return max(p.part_cells, (p.part_state[0] + kSplitParts - 1) / kSplitParts);
+    const uint32_t total = p.part_state[0];
+    const uint32_t g = min(p.part_cells, max(p.part_cells_least, (total + kFillParts - 1) / kFillParts));
+    return p.many_parts ? max(g, (total + kSplitParts - 1) / kSplitParts) : g;
 }
 
 // The parts of every meshlet (one for a meshlet that shows nowhere: it writes
@@ -523,8 +529,11 @@ __global__ void __launch_bounds__(256) k_list_parts(DiffParams p) {
 constexpr uint32_t kRoundRuns = 128;
 constexpr uint32_t kPartBlocks = 256;
 
-// Cells of a part where they are few enough (part_cells)
-uint32_t part_cells_least(uint32_t cell_blocks) { return std::max(1u, kPartBlocks / cell_blocks); }
+// Cells of a whole part, and the least of one (part_cells)
+uint32_t whole_part_cells(const DiffParams& p) { return std::max(1u, kPartBlocks / p.cell_blocks); }
+uint32_t least_part_cells(const DiffParams& p) {
+    return p.m.count < kFillParts ? std::max(1u, whole_part_cells(p) / 4) : whole_part_cells(p);
+}
 
 __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* s_wave, uint32_t& total) {
     const uint32_t lane = __lane_id(), wid = threadIdx.x >> 6;
@@ -958,11 +967,14 @@ hipError_t sum_texels(DiffWorkspace& w, const uint32_t* keys, uint32_t n, uint32
 
 namespace {
 
-// Parts the meshlets can have beyond one each: none where the cells of all
-// views make one part (up to 256x256 pixels), kSplitParts at most.
+// Parts the meshlets can have beyond one each, kSplitParts at most: with parts
+// of whole_part_cells, or up to kFillParts smaller ones. None where the cells
+// of all views make one part.
 uint32_t split_parts(const DiffParams& p) {
-    const size_t group = part_cells_least(p.cell_blocks), cells = (size_t)p.num_views * p.cell_words * 32;
-    return (uint32_t)std::min<size_t>(p.m.count * ((cells + group - 1) / group - 1), kSplitParts);
+    const size_t cells = (size_t)p.num_views * p.cell_words * 32;
+    auto extra = [&](size_t group) { return (size_t)p.m.count * ((cells + group - 1) / group - 1); };
+    return (uint32_t)std::max(std::min<size_t>(extra(whole_part_cells(p)), kSplitParts),
+                              std::min<size_t>(extra(least_part_cells(p)), kFillParts));
 }
 
 size_t cell_mark_words(const DiffParams& p) { return (size_t)p.num_views * p.m.count * p.cell_words; }
@@ -1061,7 +1073,8 @@ hipError_t launch_diff_backward(DiffParams p, DiffWorkspace& w, uint64_t num_tex
     p.parts = w.part_list;
     p.part_sums = w.part_sums;
     p.many_parts = split_parts(p) == kSplitParts;
-    p.part_cells = part_cells_least(p.cell_blocks);
+    p.part_cells = whole_part_cells(p);
+    p.part_cells_least = least_part_cells(p);
     p.block_runs = w.block_runs;
     p.run_mesh = w.run_mesh;
     p.run_tri = w.run_tri;
