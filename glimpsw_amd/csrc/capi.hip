@@ -703,29 +703,33 @@ struct LaunchShape {
     uint32_t raster_threads = 256;
 };
 
-// Bin capacity of a draw that names none: the lists of all its bins take
-// about 16 MiB where that is more than 1,024 entries each, so a small frame
-// of many meshlets keeps its records in the lists. What is past the capacity
-// goes to the overflow pass, where a wave walks each triangle over the whole
-// frame: 10,331 meshlets at 180x156 (120 bins, 3,600 entries each on average)
-// took 457 us with 1,024 entries a bin, 345 of it the overflow, and take 180.
-// A frame of fewer than kFewBins bins keeps 1,024: its bins' blocks would walk
-// everything while the rest of the card is idle, and the overflow's triangles
-// are small there. 20,000 meshlets of the same density, with 1,024 entries and
-// with longer lists: 1 bin 95 and 820 us, 4 bins 110 and 311, 16 bins 135 and
-// 139, 48 bins 194 and 103; over seven scenes the lines cross between 20 and 36.
-// The overdraw and deferred pipelines (`layers`) walk a bin's list more slowly
-// and their overflow 64 records a wave: in few bins they keep a short list
-// where it would overflow anyway, else the long one. Overdraw of 20,000
-// meshlets in 1 and 16 bins with 64, 1,024 and all entries: 133, 205, 2,847
-// and 369, 452, 561 us; of 3,000: 81, 161, 658 and 313, 173, 173.
+// Bin capacity of a draw that names none. A record past it goes to the
+// overflow pass, where a wave walks each triangle over the whole frame, while
+// a bin's list is one block's work from end to end (about 22 ns a record): long
+// lists pay where the records spread over many bins, short ones where few bins
+// hold most of them. So a bin holds 1,024 entries more than the draw has
+// meshlets (a bin of a frame that they cover evenly gets 0.1 to 1 record a
+// meshlet), up to 16 MiB of lists. Times with 1,024 entries, with this rule
+// and with all 16 MiB: 12,000 meshlets in eight layers at 180x156 569, 205 and
+// 205 us, 4,000 of them 157, 98, 98; 1,000 in a cluster over a tenth of that
+// height 91, 109, 460, 4,000 213, 290, 845.
+// In fewer than kFewBins bins, or one or two rows of them, most blocks are idle
+// in any case and the overflow's triangles are small: 20,000 meshlets with
+// 1,024 entries and with all: 1 bin 95 and 820 us, 16 bins 135 and 139, 52 bins
+// in a row 493 and 2,042 (37,000 meshlets), but 48 bins of 128x96 194 and 103.
+// The overdraw and deferred pipelines (`layers`) walk a list more slowly and
+// their overflow 64 records a wave: in few bins they keep lists that hold
+// everything, or 64 entries where nothing would do: overdraw of 20,000
+// meshlets in 1 and 16 bins with 64, 1,024 and all entries 133, 205, 2,847 and
+// 369, 452, 561 us; of 3,000 81, 161, 658 and 313, 173, 173.
 constexpr uint64_t kListEntries = 1ull << 22;
-constexpr uint64_t kFewBins = 24;
-uint32_t default_bin_capacity(uint64_t bins, uint64_t meshlets, bool layers) {
-    if (bins < kFewBins && !layers) return LaunchShape().bin_capacity;
-    if (bins < kFewBins && (bins <= 2 || meshlets > 512 * bins)) return 64;
-    const uint64_t room = kListEntries / std::max<uint64_t>(bins, 1) / 64 * 64;
-    return (uint32_t)std::max<uint64_t>(LaunchShape().bin_capacity, std::min(room, meshlets * 128));
+constexpr uint32_t kFewBins = 24, kFewBinEntries = 2048;
+uint32_t default_bin_capacity(uint32_t bins_x, uint32_t bins_y, uint64_t meshlets, bool layers) {
+    const uint64_t bins = (uint64_t)bins_x * bins_y, least = LaunchShape().bin_capacity;
+    if (layers && bins < kFewBins) return bins <= 2 || meshlets > 512 * bins ? 64 : kFewBinEntries;
+    if (bins < kFewBins || std::min(bins_x, bins_y) <= 2) return (uint32_t)least;
+    const uint64_t room = kListEntries / bins / 64 * 64;
+    return (uint32_t)std::max(least, std::min(room, least + meshlets));
 }
 
 // Clipped triangles are rare (the reference measures < 0.1%, README.md:93);
@@ -795,13 +799,15 @@ ListEntries list_entries(const BinTotals& bins, size_t bin_capacity, size_t reco
 // Lists to allocate for a draw with the default capacity: what a draw of no
 // more meshlets into any framebuffer no larger in either direction needs, so
 // that after the largest draw none allocates (a stream that is being captured
-// must not). A smaller framebuffer's bins hold more entries each: up to
+// must not). A smaller framebuffer's bins can hold more entries each: up to
 // kListEntries in all, and its coarser bins, from kRectBins bins on, no more
 // than that together.
 ListEntries default_list_entries(const BinTotals& bins, size_t bin_capacity, size_t meshlets, size_t record_slots) {
     ListEntries n = list_entries(bins, bin_capacity, record_slots);
+    n.fine = std::max<size_t>(n.fine, kFewBins * kFewBinEntries);
     if (bins.bins >= kFewBins)
-        n.fine = std::max<size_t>(n.fine, std::min<size_t>(bins.bins * meshlets * 128, kListEntries));
+        n.fine = std::max<size_t>(n.fine, std::min<size_t>(bins.bins * (meshlets + LaunchShape().bin_capacity),
+                                                           kListEntries));
     const size_t most = list_entries(bins, kListEntries / kRectBins, record_slots).coarse;
     n.coarse = std::max<size_t>(n.coarse, std::min<size_t>(most, kListEntries));
     return n;
@@ -990,7 +996,7 @@ int glimp_draw_meshlets(glimp_context* c, glimp_framebuffer* f, glimp_scene* s, 
     const BinTotals bins = direct ? BinTotals() : layout_bins(views, sh.bin_size);
     const bool alpha = (s->has_alpha && !overdraw) || deferred;    // FS_Overdraw has no alpha test
     const bool default_capacity = layers || !d->bin_capacity;
-    if (default_capacity) sh.bin_capacity = default_bin_capacity(bins.bins, d->meshlet_count, layers);
+    if (default_capacity) sh.bin_capacity = default_bin_capacity(views[0].bins_x, views[0].bins_y, d->meshlet_count, layers);
     const size_t clipq = clip_capacity_for(d->meshlet_count);
     int rc = prepare_scratch(c->draw_scratch, d->meshlet_count, clipq, bins, sh, !direct, alpha, default_capacity);
     if (rc != GLIMP_OK) return rc;

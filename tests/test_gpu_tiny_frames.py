@@ -1,8 +1,8 @@
 """Frames of few screen bins and many meshlets, on both sides of the sizes at
-which a draw's default lists change (2, 4 and 24 bins, 512 meshlets a bin), so
-that most records are drawn from the bins or most from the overflow list. All
-three pipelines, two draws on one clear; layers equal the oracle's bit for
-bit."""
+which a draw's default lists change (2, 4 and 24 bins, two bin rows, 512
+meshlets a bin), so that most records are drawn from the bins or most from the
+overflow list. All three pipelines, two draws on one clear; layers equal the
+oracle's bit for bit."""
 import pytest
 
 import oracle
@@ -28,6 +28,8 @@ def scene():
     (32, 32, 2049),
     (92, 52, 2200),          # 24 bins
     (92, 48, 2200),          # 18 bins
+    (336, 32, 2200),         # two rows of 21 bins
+    (336, 36, 2200),         # three
 ])
 def test_layers_match_oracle(gpu_ctx, scene, pipeline, width, height, count):
     import glimpsw_amd as g
