@@ -43,7 +43,7 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 # Vector-ALU issue rate: 256 CUs x 4 SIMDs, one wave64 VALU instruction per
 # four cycles of a 16-lane SIMD at the 2.4 GHz peak clock (part of the
-# instructions issue faster: the lit resolve retires 735 G/s).
+# instructions issue faster: the lit resolve retires 750 G/s).
 VALU_PEAK_WAVE_INSTS = 256 * 4 * 2.4e9 / 4
 
 
@@ -529,7 +529,9 @@ def main() -> int:
     # The lit resolve alone: `steps` back-to-back launches over the vis-buffer
     # the frame left, between two events on the stream it runs on. The
     # per-dispatch events above stamp each dispatch with extra packets that
-    # add a few microseconds to every kernel; this loop does not.
+    # add a few microseconds to every kernel; this loop does not, but where a
+    # call takes the host longer than the kernel runs (few steps on a slow
+    # host) it times the host.
     resolve_us = None
     if not args.direct:
         resolve = lambda: fb.resolve(ds, view.object_to_clip, g.GLIMP_RESOLVE_LIT, lighting, stream)  # noqa: E731
@@ -588,11 +590,12 @@ def main() -> int:
                             "valu": _valu_roofline(traffic, name, avg_us)}
     dom = max(kern.items(), key=lambda kv: kv[1][1])[0]
     dk = per_kernel[dom]
-    # the roofline's duration: the dominant kernel's own back-to-back loop
-    # where it has one (the lit resolve), else its dispatch-stamped average
+    # the roofline's duration: the dispatch-stamped average of the dominant
+    # kernel, or its own back-to-back loop where it has one (the lit resolve)
+    # and that is shorter; both can only add to the kernel's time
     roof_us, roof_timing = dk["avg_us"], ("dispatch-stamped events (hipExtLaunchKernel) over the timed steps of "
                                           "the eager frame at the headline shape")
-    if dom == "resolve_lit" and resolve_us:
+    if dom == "resolve_lit" and resolve_us and resolve_us < roof_us:
         roof_us = resolve_us
         roof_timing = (f"{args.steps} back-to-back launches of the frame's lit resolve between two events on its "
                        "stream")

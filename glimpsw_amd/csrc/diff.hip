@@ -521,7 +521,7 @@ __global__ void __launch_bounds__(256) k_list_parts(DiffParams p) {
 // One part a block at a time: the runs of its cells' pixel blocks, 256 blocks
 // at a time, are listed in block order and taken in rounds of kRoundRuns:
 // their sums are staged in LDS, each triangle's are a bit mask, and a thread
-// per (triangle, sum) adds them in order. 2.76 M pixels, 6,000 meshlets: 137 us
+// per (triangle, sum) adds them in order. 2.76 M pixels, 6,000 meshlets: 121 us
 // (sorting and reducing 8.3 M vertex records took 574), most of it the
 // meshlets at the eye, whose parts list thousands of runs; one block per
 // meshlet took 360 us with a linear search for the runs and a thread per
@@ -797,8 +797,8 @@ struct CellSum {
 
 // One thread per run piece of a tile of kTile sorted records: 111 us for 2.76 M
 // records, bound by the gather of 32 bytes a record in texel order. With the
-// sort (140 us, 2.76 M keys instead of 11 M) and the corners (47 us) the
-// texel gradients take 298 us, 504 before.
+// sort (125 us, 2.76 M keys instead of 11 M) and the corners (48 us) the
+// texel gradients take 289 us, 504 before.
 // Corner: every corner of a cell (kWholeCells), or one of them alone, by its
 // own texel.
 constexpr int kWholeCells = -1;

@@ -2875,7 +2875,7 @@ __device__ __forceinline__ void gbuffer_fragment(const DrawParams& p, const Appr
 // has its alpha record.
 //
 // One block per bin walks the bin's records again: 960x540, 36,600 records of
-// which some cover much of the view, 76 us beside a 43 us bin raster. Waves
+// which some cover much of the view, 52 us beside a 41 us bin raster. Waves
 // of 64 records each, walking all their tiles with global atomics and then
 // again for the G-buffer, took 1,477 and 2,297 us: a view-sized triangle was
 // one wave's work. After a clear the pass also writes the clear colour where

@@ -16,12 +16,13 @@
 // min filter, Texture.h:432) and the per-light early-outs. A 64-lane wave
 // holds four tiles, so those decisions are ballots over 16-lane groups.
 //
-// Bound by vector instructions (eight waves per SIMD, a tenth of the memory
-// bandwidth). The surface's inputs come in gathered form (DevMeshlets): one
-// load per vertex, the triangle's corners in one word and the normals already
-// unpacked, where each pixel unpacked and normalised its triangle's three
-// (1080p lit frame 54 -> 46 us, four 2880x1620 views 536 -> 444 us, with
-// normal maps 98 -> 77 us at 2044x1412).
+// Bound by vector instructions (eight waves per SIMD, an eighth of the memory
+// bandwidth) since the reciprocal tables are in LDS; before that by their
+// gathers through the L1. The surface's inputs come in gathered form
+// (DevMeshlets): one load per vertex, the triangle's corners in one word and
+// the normals already unpacked, where each pixel unpacked and normalised its
+// triangle's three (1080p lit frame 54 -> 46 us, four 2880x1620 views 536 ->
+// 444 us, with normal maps 98 -> 77 us at 2044x1412).
 #include <hip/hip_runtime.h>
 
 #include "internal.h"
